@@ -353,7 +353,7 @@ def decode_workload(timer, lens, args, with_uniform, seed=11, nosplit=False):
          "decode_kernel_us": dec_us, "merge_kernel_us": mrg_us,
          "kernel_launches": k, "kv_copies": ncopy, "workgroups": info.workgroups,
          "split_pairs": info.split_pairs, "paired": info.paired,
-         "decode_kernel": "decode_pair_kernel" if info.paired else "decode_balanced_kernel"}
+         "decode_kernel": "decode_balanced_kernel"}
     if with_uniform:
         mu = statistics.median(times[1])
         r["uniform"] = {"us_per_step": round(mu * 1e3, 2), "chunks": nc,
@@ -668,11 +668,7 @@ def tree_workload(timer, args):
 
 TIMELINE_LIB = os.path.join(ROOT, "cuda-kernel-lab_amd", "lib", "timeline", "libpdattn.so")
 TL_ROWS, TL_SLOTS = 8192, 32          # the stamp table of csrc/timeline.h
-DECODE_STAMPS = ([(0, "start"), (1, "descriptors staged"), (2, "q rows staged"), (3, "first ring step")]
-                 + [(4 + 2 * s, f"segment {s} streamed") for s in range(12)]
-                 + [(5 + 2 * s, f"segment {s} flushed") for s in range(12)] + [(31, "done")])
-# the paired kernel's stamp 2: its first page read back from LDS (q pieces go to registers)
-PAIR_STAMPS = ([(0, "start"), (1, "descriptors staged"), (2, "first page in registers"), (3, "first ring step")]
+DECODE_STAMPS = ([(0, "start"), (1, "descriptors staged"), (2, "first loads next"), (3, "first block computed")]
                  + [(4 + 2 * s, f"segment {s} streamed") for s in range(12)]
                  + [(5 + 2 * s, f"segment {s} flushed") for s in range(12)] + [(31, "done")])
 PREFIX_STAMPS = ([(0, "start"), (1, "ids staged"), (2, "block 0 in LDS")]
@@ -736,10 +732,9 @@ def timeline(args):
         bt, t = make_device_batch(lens, 32, 8, seed=11)
         fn, plan, ws = plan_runner(bt, t, s)
         info = plan.info()
-        W = info.workgroups // 2 if info.paired else info.workgroups   # workgroups of the launch
-        stamps = PAIR_STAMPS if info.paired else DECODE_STAMPS
-        print(json.dumps({"timeline": args.timeline, "kernel": "decode_pair_kernel" if info.paired
-                          else "decode_balanced_kernel", "launch_workgroups": W}), flush=True)
+        W = info.workgroups   # (the launch's workgroups, one or two of these each: rows past them hold no stamp)
+        stamps = DECODE_STAMPS
+        print(json.dumps({"timeline": args.timeline, "kernel": "decode_balanced_kernel", "plan_workgroups": W}), flush=True)
         reset("decode")
         runs = []
         for _ in range(reps):

@@ -254,10 +254,11 @@ struct pdattn_plan {
     int64_t U = 0;
     int split_pairs = 0, max_contrib = 0, n_entries = 0, n_slots = 0, segments = 0;
     int cmax = 0;                     // > 0: partial slots laid out by merge entry (e * cmax + k)
-    bool pair = false;                // page-range plan run by the paired kernel (W / 2 workgroups)
+    int hp = 1;                       // kv heads per kernel workgroup (W / hp workgroups)
     // workspace layout (bytes from the base)
     size_t off_desc = 0, off_list = 0, off_plse = 0, off_po = 0, ws_bytes = 0;
-    std::vector<int32_t> host_blob;   // desc[W * kBalDescInts] followed by the merge list
+    int stride = 8;                   // ints per descriptor block
+    std::vector<int32_t> host_blob;   // desc[W * stride] followed by the merge list
     void* pinned = nullptr;           // pinned copy of host_blob for stream-ordered upload
     size_t blob_bytes = 0;
     uint64_t id = new_owner();        // owner of its uploaded schedules (resident-schedule records)
@@ -312,13 +313,12 @@ namespace {
 // grows (doubling) until every workgroup has at most seg_cap (<= kSegMax) segments and kRangeMax
 // pages.
 int build_balanced_plan(const int32_t* indptr, const int32_t* last, int B, int Hq, int Hkv,
-                        int force_wg, int chunk_pages, bool merge_all, pdattn_plan* pl,
-                        int seg_cap = 0, bool pairable = false) {
+                        int force_wg, int chunk_pages, bool merge_all, pdattn_plan* pl) {
     int G = 0;
     if (int st = check_heads(Hq, Hkv, &G)) return st;
-    // at G = 8 the decode kernel stages q rows for at most kStepSegMax segments per workgroup
-    const bool wide = G > 4;
-    if (seg_cap <= 0) seg_cap = wide ? kStepSegMax : kSegMax;
+    const int seg_cap = kSegMax;
+    // (a cascade's suffix runs beside the prefix workgroups with a shorter LDS page list)
+    const int range_cap = merge_all ? kStepRangeMax : kRangeMax;
     if (B < 0) return fail(PDATTN_ERR_INVALID_ARGUMENT, "B=%d is negative", B);
     if (chunk_pages < 0 || chunk_pages > kRangeMax)
         return fail(PDATTN_ERR_INVALID_ARGUMENT, "chunk_pages=%d outside [0, %d]", chunk_pages, kRangeMax);
@@ -334,19 +334,23 @@ int build_balanced_plan(const int32_t* indptr, const int32_t* last, int B, int H
     pl->nnz = B > 0 ? indptr[B] - indptr[0] : 0;
     pl->U = (int64_t)Hkv * pl->nnz;
 
-    // grid: one workgroup per CU (the kernel's four waves take one SIMD each; two at G = 8), never more
-    // workgroups than page units; a forced size needs no device query
+    // grid: one kernel workgroup per CU (its four waves take one SIMD each); a forced size needs no
+    // device query. A default page-range plan of an even Hkv runs two plan workgroups (neighbouring
+    // kv heads of one range) per kernel workgroup: 512 contiguous bytes of every token row are then
+    // read together, which streams faster (64 ragged sequences of 256-4096 tokens, G = 4: 93.7 us one
+    // head per workgroup, 89.8 us two, 92.3 us four; G = 8: 98.0, 93.5, 97.9 us). Not below 8 pages
+    // per range, where the merge's twice as many partials cost more (one sequence of 4096 tokens 8.91
+    // against 9.22 us, of 16384 16.43 against 16.36), unless the sequences are more than the ranges of
+    // one head per workgroup (40 sequences of 94-988 tokens 25.0 against 21.9 us).
     int64_t W = force_wg;
-    // The paired kernel (two kv heads per workgroup, pages staged in LDS) runs a default page-range
-    // plan at G <= 4 with an even Hkv: two plan workgroups per CU, one kernel workgroup.
-    const bool pair = pairable && force_wg <= 0 && chunk_pages == 0 && !merge_all && !wide &&
-                      Hkv % 2 == 0;
+    int hp = 1;
     if (W <= 0) {
         DeviceFacts f;
         if (int st = device_facts(&f)) return st;
-        // G = 8 (VALU-limited per page): two workgroups per CU, except for the cascade's suffix,
-        // whose workgroups share the CUs with the prefix pass
-        W = (int64_t)f.cus * (wide && !merge_all ? 2 : 1) * (pair ? 2 : 1);
+        const int64_t W2 = (int64_t)f.cus * 2;
+        if (chunk_pages == 0 && Hkv % 2 == 0 && W2 >= Hkv && W2 % Hkv == 0 && (pl->nnz >= 8 * (W2 / Hkv) || B > f.cus / Hkv))
+            hp = 2;
+        W = (int64_t)f.cus * hp;
     }
     // Page-range groups, the default: the pages of all sequences, in page-table order, are cut
     // into NG = W / Hkv equal ranges, and workgroup g * Hkv + h takes range g for kv head h. The
@@ -357,7 +361,7 @@ int build_balanced_plan(const int32_t* indptr, const int32_t* last, int B, int H
     const bool grouped = chunk_pages == 0 && W >= Hkv && W % Hkv == 0;
     if (!grouped) {
         W = std::max<int64_t>(1, std::min<int64_t>(W, std::max<int64_t>(1, pl->U)));
-        W = std::max<int64_t>(W, (pl->U + kRangeMax - 1) / kRangeMax);
+        W = std::max<int64_t>(W, (pl->U + range_cap - 1) / range_cap);
     }
     if (W > (1 << 28)) return fail(PDATTN_ERR_INVALID_ARGUMENT, "grid too large");
 
@@ -367,44 +371,37 @@ int build_balanced_plan(const int32_t* indptr, const int32_t* last, int B, int H
     const int jbase = pl->jbase;
     auto seq_len = [&](int b) { return (indptr[b + 1] - indptr[b] - 1) * kPage + last[b]; };
     const size_t pairs = (size_t)B * Hkv;
-    struct SegRef { int64_t w; int idx; size_t pair; };
-    std::vector<int32_t> desc;
+    struct SegRef { int64_t w; int idx; size_t pair; int32_t f[kSegInts]; };
+    std::vector<int> wsegs;       // segments of each workgroup
     std::vector<SegRef> refs;
     std::vector<int> nc;
     // appends segment {b, kvh, pages [p0, p1) of sequence b} to workgroup w, whose page list starts
     // at page-table position wbeg (relative to kv_indptr[0]); false when w is full
     auto add_segment = [&](int64_t w, int64_t wbeg, int b, int kvh, int p0, int p1) {
-        int32_t* d = &desc[(size_t)w * kBalDescInts];
-        if (d[0] == seg_cap) return false;
-        int32_t* sg = d + 8 + kSegInts * d[0];
+        if (wsegs[w] == seg_cap) return false;
         const int np = indptr[b + 1] - indptr[b];
         const int64_t pos = indptr[b] - jbase + p0;
-        sg[0] = b;
-        sg[1] = kvh;
-        sg[2] = (int)(pos - wbeg);
-        sg[3] = p1 - p0;
-        sg[4] = p0 * kPage;
-        sg[5] = p1 == np ? seq_len(b) : p1 * kPage;
-        sg[6] = (int)pos;
-        sg[7] = -1;
         const size_t pr = (size_t)b * Hkv + kvh;
-        refs.push_back({w, d[0], pr});
+        refs.push_back({w, wsegs[w]++, pr,
+                        {b, kvh, (int)(pos - wbeg), p1 - p0, p0 * kPage, p1 == np ? seq_len(b) : p1 * kPage, (int)pos, -1}});
         ++nc[pr];
-        ++d[0];
         return true;
     };
     if (grouped) {
         int64_t NG = std::min<int64_t>(W / Hkv, std::max<int64_t>(1, nnz));
+        // (default grid: a range shorter than a page for each of a head's four waves only adds partials
+        // to merge, unless it keeps short sequences in ranges of their own)
+        if (force_wg <= 0) NG = std::min<int64_t>(NG, std::max<int64_t>({(int64_t)1, (int64_t)B, (nnz + 3) / 4}));
         for (;;) {
             W = NG * Hkv;
-            desc.assign((size_t)W * kBalDescInts, 0);
+            wsegs.assign((size_t)W, 0);
             refs.clear();
             nc.assign(pairs, 0);
             bool ok = true;
             int b = 0;
             for (int64_t g = 0; g < NG && ok; ++g) {
                 const int64_t lo = nnz * g / NG, hi = nnz * (g + 1) / NG;
-                if (hi - lo > kRangeMax) { ok = false; break; }
+                if (hi - lo > range_cap) { ok = false; break; }
                 while (b < B && indptr[b + 1] - jbase <= lo) ++b;   // first sequence reaching past lo
                 for (int bb = b; bb < B && indptr[bb] - jbase < hi && ok; ++bb) {
                     const int64_t s0 = std::max<int64_t>(lo, indptr[bb] - jbase);
@@ -420,10 +417,10 @@ int build_balanced_plan(const int32_t* indptr, const int32_t* last, int B, int H
         }
         pl->P = (int)((nnz + W / Hkv - 1) / (W / Hkv));   // pages per range
         pl->ngroups = (int)(W / Hkv);
-        pl->pair = pair;   // (W = NG Hkv is even: plan workgroups 2 x and 2 x + 1 share range g)
+        pl->hp = hp;   // (W = NG Hkv is even: plan workgroups 2 x and 2 x + 1 share range g)
     }
     for (; !grouped;) {
-        desc.assign((size_t)W * kBalDescInts, 0);
+        wsegs.assign((size_t)W, 0);
         refs.clear();
         nc.assign(pairs, 0);
         bool ok = true;
@@ -440,24 +437,15 @@ int build_balanced_plan(const int32_t* indptr, const int32_t* last, int B, int H
                             wbeg = wend;
                             wend = U * (w + 1) / W;
                         }
-                        if (wend - wbeg > kRangeMax) { ok = false; break; }
+                        if (wend - wbeg > range_cap) { ok = false; break; }
                         const int take = (int)std::min<int64_t>(pn - done, wend - u);
-                        int32_t* d = &desc[(size_t)w * kBalDescInts];
-                        if (d[0] == seg_cap) { ok = false; break; }
-                        int32_t* sg = d + 8 + kSegInts * d[0];
+                        if (wsegs[w] == seg_cap) { ok = false; break; }
                         const int p0 = pa + done, p1 = pa + done + take;
-                        sg[0] = b;
-                        sg[1] = kvh;
-                        sg[2] = (int)(u - wbeg);
-                        sg[3] = take;
-                        sg[4] = p0 * kPage;
-                        sg[5] = p1 == np ? seq_len(b) : p1 * kPage;
-                        sg[6] = indptr[b] - pl->jbase + p0;
-                        sg[7] = -1;
                         const size_t pr = (size_t)b * Hkv + kvh;
-                        refs.push_back({w, d[0], pr});
+                        refs.push_back({w, wsegs[w]++, pr,
+                                        {b, kvh, (int)(u - wbeg), take, p0 * kPage, p1 == np ? seq_len(b) : p1 * kPage,
+                                         indptr[b] - pl->jbase + p0, -1}});
                         ++nc[pr];
-                        ++d[0];
                         u += take;
                         done += take;
                     }
@@ -503,9 +491,19 @@ int build_balanced_plan(const int32_t* indptr, const int32_t* last, int B, int H
     } else {
         cmax = 0;
     }
+    // descriptor blocks: 8 ints of header and the segments, as many ints each as the fullest needs
+    int most = 0;
+    for (int n : wsegs) most = std::max(most, n);
+    const int stride = 8 + kSegInts * most;
+    std::vector<int32_t> desc((size_t)W * stride, 0);
+    for (int64_t w = 0; w < W; ++w) {
+        desc[(size_t)w * stride] = wsegs[w];
+        desc[(size_t)w * stride + 1] = pl->tag;
+    }
     std::vector<int> seen(pairs, 0);
     for (const SegRef& rf : refs) {
-        int32_t* sg = &desc[(size_t)rf.w * kBalDescInts + 8 + kSegInts * rf.idx];
+        int32_t* sg = &desc[(size_t)rf.w * stride + 8 + kSegInts * rf.idx];
+        std::memcpy(sg, rf.f, sizeof rf.f);
         const int k = seen[rf.pair]++;
         if (need_slots(rf.pair)) sg[7] = slot0[rf.pair] + k;
     }
@@ -517,13 +515,13 @@ int build_balanced_plan(const int32_t* indptr, const int32_t* last, int B, int H
     pl->n_slots = slots;
     pl->cmax = cmax;
     pl->segments = (int)refs.size();
-    for (int64_t w = 0; w < W; ++w) desc[(size_t)w * kBalDescInts + 1] = pl->tag;
-    pl->host_blob = desc;
+    pl->stride = stride;
+    pl->host_blob = std::move(desc);
     pl->host_blob.insert(pl->host_blob.end(), {pl->tag, pl->n_entries, cmax, 0});   // list header
     pl->host_blob.insert(pl->host_blob.end(), list.begin(), list.end());
 
     size_t off = 0;
-    pl->off_desc = off;  off += align_up(sizeof(int32_t) * desc.size());
+    pl->off_desc = off;  off += align_up(sizeof(int32_t) * (size_t)W * stride);
     pl->off_list = off;  off += align_up(sizeof(int32_t) * (4 + list.size()));
     pl->off_plse = off;  off += align_up(sizeof(float) * std::max(1, slots) * G);
     pl->off_po = off;    off += align_up(sizeof(float) * std::max(1, slots) * G * kHeadDim);
@@ -540,6 +538,10 @@ void free_plan_storage(pdattn_plan* pl) {
     }
 }
 
+// Ints of a plan's schedule as pdattn_plan_get_schedule gives it.
+size_t schedule_ints(const pdattn_plan* pl) {
+    return (size_t)pl->W * kBalDescInts + 4 * (size_t)(1 + pl->n_entries);
+}
 // Bytes of a plan's schedule in its workspace (descriptors and merge list; the partial slots
 // after them are scratch of each run).
 size_t schedule_bytes(const pdattn_plan* pl) { return pl->off_plse - pl->off_desc; }
@@ -549,7 +551,7 @@ int upload_plan(pdattn_plan* pl, void* ws, size_t bytes, hipStream_t s) {
     if (bytes < pl->ws_bytes)
         return fail(PDATTN_ERR_WORKSPACE, "workspace holds %zu bytes, plan needs %zu", bytes, pl->ws_bytes);
     char* base = static_cast<char*>(ws);
-    const size_t desc_bytes = sizeof(int32_t) * (size_t)pl->W * kBalDescInts;
+    const size_t desc_bytes = sizeof(int32_t) * (size_t)pl->W * pl->stride;
     if (pl->blob_bytes && !pl->pinned) {
         // pinned staging copy, made once: the copies below are stream-ordered and asynchronous
         hipError_t e = hipHostMalloc(&pl->pinned, pl->blob_bytes, hipHostMallocDefault);
@@ -587,7 +589,14 @@ BalArgs bal_args(const pdattn_plan* pl, const void* q, const void* k, const void
     a.ngroups = pl->ngroups;
     a.nnz = pl->nnz;
     a.tag = pl->tag;
+    a.desc_stride = pl->stride;
     a.qrow_b = pl->ngroups > 0 && pl->B == 1 ? 0 : -1;
+    if (pl->ngroups > 0) {
+        a.range_q = (uint32_t)(pl->nnz / pl->ngroups);
+        a.range_r = (uint32_t)(pl->nnz % pl->ngroups);
+        a.range_m = 0xFFFFFFFFu / (uint32_t)pl->ngroups;
+        a.hkv_m = 0xFFFFFFFFu / (uint32_t)pl->Hkv;
+    }
     return a;
 }
 
@@ -619,7 +628,7 @@ int run_plan(const pdattn_plan* pl, const void* q, const void* k, const void* v,
     res_written_outputs(out, lse, (size_t)pl->B * pl->Hq);
     if (pl->U > 0 && decode) {
         const BalArgs a = bal_args(pl, q, k, v, indices, sm_scale, out, lse, base);
-        if (pl->pair) PD_HIP(launch_decode_pair(a, pl->G, s));
+        if (pl->hp > 1) PD_HIP(launch_decode_pair(a, pl->G, s));
         else PD_HIP(launch_decode_balanced(a, pl->G, s));
     }
     if (join) PD_HIP(hipStreamWaitEvent(s, join, 0));
@@ -959,13 +968,14 @@ static int launch_uniform_split(const PartialArgs& a, int G, hipStream_t s) {
     }
     DeviceFacts f;
     if (int st = device_facts(&f)) return st;
-    const int64_t n_items = (int64_t)a.num_chunks * a.B * a.Hkv;
+    // An item is one chunk of hp kv heads: two where that still fills the CUs (8 x 8192 tokens in 4
+    // chunks, 256 items of one head or 128 of two: 47.9 against 54.1 us).
+    const int hp = a.Hkv % 2 == 0 && (int64_t)a.num_chunks * a.B * a.Hkv >= 2 * f.cus ? 2 : 1;
+    const int64_t n_items = (int64_t)a.num_chunks * a.B * (a.Hkv / hp);
     if (n_items > (int64_t)1 << 30) return fail(PDATTN_ERR_INVALID_ARGUMENT, "too many chunks");
-    // at G = 8 the kernel's compact layout holds kStepSegMax segments, two workgroups per CU
-    const bool wide = G > 4;
-    const int64_t slots = (int64_t)f.cus * (wide ? 2 : 1);
+    const int64_t slots = (int64_t)f.cus;
     int64_t per = (n_items + slots - 1) / slots;
-    per = std::max<int64_t>(1, std::min<int64_t>({per, (int64_t)(wide ? kStepSegMax : kSegMax), kRangeMax / ppi}));
+    per = std::max<int64_t>(1, std::min<int64_t>({per, (int64_t)kSegMax, kRangeMax / ppi}));
     UniArgs u;
     BalArgs& d = u.d;
     d.q = a.q;
@@ -994,7 +1004,7 @@ static int launch_uniform_split(const PartialArgs& a, int G, hipStream_t s) {
     u.chunk_base = a.chunk_base;
     u.n_items = (int)n_items;
     u.per_wg = (int)per;
-    PD_HIP(launch_decode_uniform(u, G, s));
+    PD_HIP(launch_decode_uniform(u, G, hp, s));
     return PDATTN_OK;
 }
 
@@ -1099,7 +1109,7 @@ namespace {
 // workspace, or use_uniform when the batch is past the kernel's staging (kDevMaxB sequences).
 struct DevLayout {
     bool use_uniform = false;
-    int W = 0, NG = 0;
+    int W = 0, NG = 0, hp = 1;   // W: workgroups of the launch, hp kv heads each
     int64_t span = 0;
     size_t off_prefix = 0, off_plse = 0, off_po = 0, bytes = 0;
 };
@@ -1113,18 +1123,19 @@ int dev_layout(const pdattn_decode_params* p, int G, DevLayout* L) {
     }
     DeviceFacts f;
     if (int st = device_facts(&f)) return st;
-    // one workgroup per CU (two at G = 8, as the plan path), whole groups of Hkv; more ranges if a
+    // one workgroup per CU of one kv head, or of two (as the plan path), whole groups of Hkv; more ranges if a
     // range could hold more pages than the kernel stages (kRangeMax): every sequence attends at
     // most ceil(span / 16) + 1 pages
     L->span = (int64_t)p->num_chunks * p->chunk_tokens;
     const int64_t per_seq = L->span / kPage + 2;
     const int64_t bound = (int64_t)p->B * per_seq;
-    int64_t NG = std::max<int64_t>(1, (int64_t)f.cus * (G > 4 ? 2 : 1) / p->Hkv);
+    L->hp = p->Hkv % 2 == 0 ? 2 : 1;
+    int64_t NG = std::max<int64_t>(1, (int64_t)f.cus * L->hp / p->Hkv);
     NG = std::max<int64_t>(NG, (bound + kRangeMax - 1) / kRangeMax);
     if (NG * p->Hkv > (1 << 24)) return fail(PDATTN_ERR_INVALID_ARGUMENT, "too many ranges");
     L->NG = (int)NG;
-    L->W = (int)(NG * p->Hkv);
-    const size_t slots = (size_t)2 * L->W * G;
+    L->W = (int)(NG * p->Hkv / L->hp);
+    const size_t slots = (size_t)2 * NG * p->Hkv * G;
     size_t off = 0;
     L->off_prefix = off; off += align_up(sizeof(int32_t) * (p->B + 1));
     L->off_plse = off;   off += align_up(sizeof(float) * slots);
@@ -1184,7 +1195,7 @@ int pdattn_decode_attention_balanced(const pdattn_decode_params* p, int G, int v
     a.prefix = reinterpret_cast<int32_t*>(base + L.off_prefix);
     a.span = L.span;
     a.kv_start = p->kv_start;
-    PD_HIP(launch_decode_ranges(a, G, s));
+    PD_HIP(launch_decode_ranges(a, G, L.hp, s));
     DevMergeArgs m;
     m.prefix = a.prefix;
     m.part_o = d.part_o;
@@ -1207,17 +1218,7 @@ int pdattn_plan_create(const int32_t* h_kv_indptr, const int32_t* h_kv_last_page
     if (B > 0 && !h_kv_indptr) return fail(PDATTN_ERR_INVALID_ARGUMENT, "null kv_indptr");
     pdattn_plan* pl = new pdattn_plan();
     int st = build_balanced_plan(h_kv_indptr, h_kv_last_page_len, B, Hq, Hkv, force_workgroups,
-                                 chunk_pages, false, pl, 0, true);
-    if (st == PDATTN_OK && pl->pair && pl->n_entries > 0) {
-        // The paired plan's ranges are half as long, so it splits this batch's sequences over
-        // twice as many workgroups: the merge's fan-in doubles, which costs more than the paired
-        // kernel gains (1x32K: 28.3 -> 30.8 us back to back). One kv head per workgroup instead.
-        free_plan_storage(pl);
-        delete pl;
-        pl = new pdattn_plan();
-        st = build_balanced_plan(h_kv_indptr, h_kv_last_page_len, B, Hq, Hkv, force_workgroups,
                                  chunk_pages, false, pl);
-    }
     if (st != PDATTN_OK) {
         free_plan_storage(pl);
         delete pl;
@@ -1238,16 +1239,23 @@ int pdattn_plan_get_info(const pdattn_plan* pl, pdattn_plan_info* info) {
     info->chunk_pages = pl->P;
     info->segments = pl->segments;
     info->merge_entries = pl->n_entries;
-    info->paired = pl->pair ? 1 : 0;
-    info->schedule_ints = (int)pl->host_blob.size();
+    info->paired = pl->hp > 1 && pl->G <= 4 && pl->n_entries == 0 ? 1 : 0;
+    info->schedule_ints = (int)schedule_ints(pl);
     return PDATTN_OK;
 }
 
 int pdattn_plan_get_schedule(const pdattn_plan* pl, int32_t* out, size_t count) {
     if (!pl || !out) return fail(PDATTN_ERR_INVALID_ARGUMENT, "null pointer");
-    if (count < pl->host_blob.size())
-        return fail(PDATTN_ERR_INVALID_ARGUMENT, "schedule holds %zu ints, %zu given", pl->host_blob.size(), count);
-    std::memcpy(out, pl->host_blob.data(), sizeof(int32_t) * pl->host_blob.size());
+    if (count < schedule_ints(pl))
+        return fail(PDATTN_ERR_INVALID_ARGUMENT, "schedule holds %zu ints, %zu given", schedule_ints(pl), count);
+    // (the public layout: every block PDATTN_SCHEDULE_WG_INTS long)
+    if (pl->host_blob.empty()) return PDATTN_OK;
+    const int32_t* src = pl->host_blob.data();
+    for (int w = 0; w < pl->W; ++w, src += pl->stride, out += kBalDescInts) {
+        std::memset(out, 0, sizeof(int32_t) * kBalDescInts);
+        std::memcpy(out, src, sizeof(int32_t) * pl->stride);
+    }
+    std::memcpy(out, src, sizeof(int32_t) * 4 * (1 + pl->n_entries));
     return PDATTN_OK;
 }
 
@@ -1439,9 +1447,9 @@ int pdattn_cascade_decode(pdattn_cascade_plan* cp, void* out, float* lse, pdattn
         StepArgs sa;
         sa.d = bal_args(&cp->sk, p.q, p.k_cache, p.v_cache, sidx, p.sm_scale, out, lse, skb);
         sa.p = a;
-        sa.n_dec = cp->sk.U > 0 ? cp->sk.W : 0;
+        sa.n_dec = cp->sk.U > 0 ? cp->sk.W / cp->sk.hp : 0;
         sa.n_pre = cp->n_items * p.Hkv;
-        PD_HIP(launch_cascade_step(sa, p.Hq / p.Hkv, s));
+        PD_HIP(launch_cascade_step(sa, p.Hq / p.Hkv, cp->sk.hp, s));
         return run_plan(&cp->sk, p.q, p.k_cache, p.v_cache, sind, sidx, p.kv_last_page_len, p.sm_scale,
                         out, lse, skb, cp->sk.ws_bytes, s, ppo, pplse, cp->n_extra, nullptr, false);
     }

@@ -6,34 +6,28 @@
 // as a normalized partial (o, lse), then a log-sum-exp merge of the partials.
 //
 // How it maps to CDNA4:
-//  * One workgroup body (balanced_body): 4 waves, one per SIMD and one workgroup per CU, walking
-//    a list of segments (pieces of one sequence and kv head), each wave on every 4th page, with
-//    one page ring across all of them. The plan/run path (decode_balanced_kernel) reads the list
-//    from a host-built plan; the reference-shaped uniform split (decode_uniform_kernel) builds it
-//    in the kernel from the device page table. A uniform chunk too long for the body's LDS page
-//    list runs on decode_partial_kernel, one workgroup per (sequence, kv head, chunk).
-//  * K and V rows go straight from HBM into VGPRs with 16-byte non-temporal loads: a 256-byte
-//    row (128 fp16) is read by LPR lanes, so one wave-wide load instruction reads 64/LPR rows of
-//    one page, each as whole 128-byte lines. No LDS staging is needed because every lane reads
-//    only the bytes it computes with.
-//  * Scores: each lane takes the fp16 dot product of its slice of q_h and k_j with
-//    v_dot2_f32_f16 (fp32 accumulate), then the LPR lanes of a row sum with DPP row ops
-//    (quad_perm, row_half_mirror, row_mirror), which leaves the score in every lane of the row.
-//  * Every lane therefore owns whole keys: it keeps its own online-softmax state (max, sum,
-//    output slice) over the keys it holds, so the PV product needs no cross-lane traffic. The
-//    64/LPR independent states of a wave are merged once at the end, in the VALU (DPP row_ror and
-//    v_permlane16/32_swap) or through LDS, and the waves of the workgroup through LDS.
+//  * The segment runner (decode_body.h, run_segments below): 4-wave workgroups, one per CU, each wave
+//    on one kv head and all its query heads, 32 keys at a time on fp16 MFMA, its pages staged by the
+//    wave itself with direct global->LDS loads. A workgroup walks a list of segments (pieces of
+//    sequences) for one kv head, or for two neighbouring heads of the same pages. The plan/run path
+//    (decode_balanced_kernel) reads the list from a host-built plan; the reference-shaped uniform
+//    split (decode_uniform_kernel) and the device-range drop-in (decode_ranges_kernel) build it in
+//    the kernel from the device page table; the fused cascade step runs it beside the prefix pass.
+//  * A uniform chunk too long for the runner's LDS page list runs on decode_partial_kernel, one
+//    workgroup per (sequence, kv head, chunk), on the vector unit:
+//    - K and V rows go straight from HBM into VGPRs with 16-byte non-temporal loads: a 256-byte row
+//      (128 fp16) is read by LPR lanes, so one wave-wide load instruction reads 64/LPR rows of one
+//      page, each as whole 128-byte lines; a two-page ring, one page in flight;
+//    - each lane takes the fp16 dot product of its slice of q_h and k_j with v_dot2_f32_f16, and the
+//      LPR lanes of a row sum with DPP row ops, which leaves the score in every lane of the row;
+//    - every lane keeps its own online-softmax state over the keys it holds; the 64/LPR states of a
+//      wave are merged once at the end, and the waves of the workgroup through LDS.
+//    LPR = 16 lanes per row, 4 rows per wave-wide load, each lane holding 4 rows x 8 dims of a page.
+//    Lane (r = lane / LPR, c = lane % LPR) holds rows i*RPI + r of each page and the 16-byte pieces
+//    kk*LPR + c (dims 8*(kk*LPR + c) .. +7), kk < PPL.
 //  * Softmax runs in base 2 on log2(e)-prescaled scores with v_exp_f32 / v_log_f32
-//    (exp(x) = 2^(x log2 e)); the running output is rescaled only when some lane's max grows
-//    (a wave-uniform branch), which after the first pages is rare.
-//  * Prefetch: a two-page ring in VGPRs; the loads of the next page are issued before the
-//    current page is computed.
-//
-// Lane geometry (both kernels), G = query heads per kv head: LPR = 16 lanes per 256-byte K/V row,
-// 4 rows per wave-wide load, each lane holding 4 rows x 8 dims of a page (keeps the fp32 output
-// state at 64 VGPRs at G = 8).
-// Lane (r = lane / LPR, c = lane % LPR) holds rows i*RPI + r of each page and the 16-byte pieces
-// kk*LPR + c (dims 8*(kk*LPR + c) .. +7), kk < PPL.
+//    (exp(x) = 2^(x log2 e)); the running output is rescaled only when some max grows (a
+//    wave-uniform branch), which after the first pages is rare.
 #include <math.h>
 
 #include <algorithm>
@@ -44,7 +38,7 @@
 
 PD_TIMELINE_TABLE(decode)
 
-#include "prefix_body.h"
+#include "decode_body.h"
 
 namespace pdattn {
 namespace {
@@ -75,18 +69,8 @@ __device__ __forceinline__ float dpp(float v) {
         float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
 }
 
-// Sum over the LPR lanes that share one K/V row (a DPP row is 16 lanes).
-template <int LPR>
-__device__ __forceinline__ float row_sum(float v) {
-    v += dpp<0xB1>(v);   // quad_perm [1,0,3,2]
-    v += dpp<0x4E>(v);   // quad_perm [2,3,0,1]
-    v += dpp<0x141>(v);  // row_half_mirror: the other quad of the 8-lane half row
-    if constexpr (LPR == 16) v += dpp<0x140>(v);  // row_mirror: the other half row
-    return v;
-}
-
-// row_sum of N independent values, one DPP step at a time across all of them (the same sums,
-// bitwise: each value goes through the same sequence of adds).
+// Sums over the LPR lanes that share one K/V row (a DPP row is 16 lanes) of N independent values, one
+// DPP step at a time across all of them.
 template <int LPR, int N>
 __device__ __forceinline__ void row_sum_all(float* v) {
 #pragma unroll
@@ -639,663 +623,313 @@ __global__ __launch_bounds__(kMergeThreads) void merge_split_kernel(MergeArgs a)
     merge_store(st, a.out + orow * kHeadDim, a.lse + orow);
 }
 
-// Per-segment merge scratch of the balanced kernel: the raw online-softmax state of every row
-// group of every wave (NS = waves x row groups sources), then per-source weights. o rows are
-// padded by 4 floats so that the row groups of a wave, which write the same columns, fall in
-// different LDS banks. The o rows hold HP of the G heads at a time (the flush takes G / HP passes).
-template <int G, int NS, int HP = G>
-struct BalSmem {
-    static constexpr int OP = kHeadDim + 4;
-    float m[NS][G];
-    float l[NS][G];
-    float o[NS][HP][OP];
-    float alpha[G][NS];       // exp(m_src - M) per head and source
-    float rinv[G];            // 1 / L
-    float lse[G];
-};
-
-template <class C>
-__device__ __forceinline__ void reset_state(WaveState<C>& st) {
+// The page list of the segments staged in S.sd, where it is not one range of kv_indices: item i of
+// the list is found in the segment whose range [qa, qa + npg) holds it (LDS reads only: a search
+// loop with loads in flight would wait for them at every iteration), then all ids are loaded in one
+// round trip. Ends with a barrier.
+template <class C, int LAY>
+__device__ __forceinline__ void stage_pages(const BalArgs& a, DecShared<C, LAY>& S, int nseg) {
+    constexpr int NT = C::NT, PMAX = DecShared<C, LAY>::PGMAX / NT;
+    const int tid = threadIdx.x;
+    const int* seg = S.sd[0] + 8;
+    const int npages = __builtin_amdgcn_readfirstlane(seg[(nseg - 1) * kSegInts + 2] + seg[(nseg - 1) * kSegInts + 3]);
+    const int32_t* kvi = a.kv_indices;
+    int src[PMAX];
 #pragma unroll
-    for (int h = 0; h < C::G; ++h) {
-        st.m[h] = -INFINITY;
-        st.l[h] = 0.f;
-#pragma unroll
-        for (int d = 0; d < C::DPL; ++d) st.o[h][d] = 0.f;
+    for (int k = 0; k < PMAX; ++k) {
+        const int i = tid + k * NT;
+        src[k] = -1;
+        if (i < npages) {
+            int si = 0;
+            while (si + 1 < nseg && seg[(si + 1) * kSegInts + 2] <= i) ++si;
+            src[k] = seg[si * kSegInts + 6] + (i - seg[si * kSegInts + 2]);
+        }
     }
-}
-
-// Reduction (max or sum) over the lanes that agree modulo G (G in 1, 2, 4, 8), leaving the result
-// in every one of them, in the VALU: quad permutations for lane distances 1 and 2, row
-// rotations by 8 and 4 within a 16-lane row (after which every lane of the row holds the result
-// of its class), and the row-pair swaps across rows.
-template <int G, bool MAX>
-__device__ __forceinline__ float class_reduce(float v) {
-    auto op = [](float x, float y) { return MAX ? fmaxf(x, y) : x + y; };
-    if constexpr (G == 1) v = op(v, dpp<0xB1>(v));   // quad_perm [1,0,3,2]
-    if constexpr (G <= 2) v = op(v, dpp<0x4E>(v));   // quad_perm [2,3,0,1]
-    v = op(v, dpp<0x128>(v));                        // row_ror:8
-    if constexpr (G <= 4) v = op(v, dpp<0x124>(v));  // row_ror:4
-    float x, y;
-    row_pair<false>(v, x, y);
-    row_pair<true>(op(x, y), x, y);
-    return op(x, y);
-}
-
-// End of a segment. Every row group of every wave is one source state (max, sum, output slice);
-// all of them go to LDS unmerged, one wave turns the per-source maxima into weights, and each
-// thread forms four outputs as one weighted sum over the sources, in source order. Writes the G
-// rows as the final fp16 out / lse (slot < 0) or as partial slot `slot` (normalized o, lse). The
-// raw outputs go through LDS HP heads at a time (HP = G: one pass).
-template <class C, int HP>
-__device__ __forceinline__ void flush_segment(BalSmem<C::G, C::NW * C::RPI, HP>& sm, WaveState<C>& st,
-                                              KArgPtr a, size_t row0, int slot,
-                                              int tid = threadIdx.x) {
-    constexpr int G = C::G, LPR = C::LPR, NS = C::NW * C::RPI;
-    // one wave computes the source weights: lane = s * G + h covers sources s + j * SL, j < J
-    constexpr int SL = 64 / G, J = (NS + SL - 1) / SL;
-    static_assert(NS % 4 == 0 && HP * 32 <= C::NT && G % HP == 0, "float4 passes");
-    // (tid: the thread's index among the C::NT threads that flush this state; every thread of the
-    // workgroup calls it, as it holds barriers)
-    const int lane = tid & 63, c = lane % LPR;
-    const int src = (tid >> 6) * C::RPI + lane / LPR;
-#pragma unroll
-    for (int hp = 0; hp < G / HP; ++hp) {
-#pragma unroll
-        for (int hh = 0; hh < HP; ++hh)
-#pragma unroll
-            for (int kk = 0; kk < C::PPL; ++kk) {
-                const int h = hp * HP + hh;
-                float4* dst = reinterpret_cast<float4*>(&sm.o[src][hh][(kk * LPR + c) * 8]);
-                dst[0] = make_float4(st.o[h][kk * 8 + 0], st.o[h][kk * 8 + 1], st.o[h][kk * 8 + 2], st.o[h][kk * 8 + 3]);
-                dst[1] = make_float4(st.o[h][kk * 8 + 4], st.o[h][kk * 8 + 5], st.o[h][kk * 8 + 6], st.o[h][kk * 8 + 7]);
-            }
-        if (hp == 0 && c == 0) {
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                sm.m[src][h] = st.m[h];
-                sm.l[src][h] = st.l[h];
-            }
-        }
-        __syncthreads();
-        if (hp == 0) {
-            if (tid < 64) {
-                const int s0 = tid / G, h = tid % G;
-                float mv[J];
-                float M = -INFINITY;
-#pragma unroll
-                for (int j = 0; j < J; ++j) {
-                    const int s = s0 + j * SL;
-                    mv[j] = s < NS ? sm.m[s][h] : -INFINITY;
-                    M = fmaxf(M, mv[j]);
-                }
-                M = class_reduce<G, true>(M);
-                float L = 0.f;
-#pragma unroll
-                for (int j = 0; j < J; ++j) {
-                    const int s = s0 + j * SL;
-                    const float al = (mv[j] == -INFINITY) ? 0.f : fast_exp2(mv[j] - M);
-                    if (s < NS) {
-                        sm.alpha[h][s] = al;
-                        L = fmaf(al, sm.l[s][h], L);
-                    }
-                }
-                L = class_reduce<G, false>(L);
-                if (tid < G) {
-                    sm.rinv[h] = L > 0.f ? 1.f / L : 0.f;
-                    sm.lse[h] = L > 0.f ? (M + fast_log2(L)) * kLn2 : -INFINITY;
-                }
-            }
-            __syncthreads();
-        }
-        if (tid < HP * 32) {
-            const int hh = tid / 32, h = hp * HP + hh, d0 = 4 * (tid % 32);
-            float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int s4 = 0; s4 < NS; s4 += 4) {
-                const float4 al = *reinterpret_cast<const float4*>(&sm.alpha[h][s4]);
-                const float alv[4] = {al.x, al.y, al.z, al.w};
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const float4 ov = *reinterpret_cast<const float4*>(&sm.o[s4 + u][hh][d0]);
-                    O.x = fmaf(alv[u], ov.x, O.x);
-                    O.y = fmaf(alv[u], ov.y, O.y);
-                    O.z = fmaf(alv[u], ov.z, O.z);
-                    O.w = fmaf(alv[u], ov.w, O.w);
-                }
-            }
-            const float ri = sm.rinv[h];
-            O.x *= ri;
-            O.y *= ri;
-            O.z *= ri;
-            O.w *= ri;
-            if (slot < 0) {
-                typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-                const h4 hv = {(_Float16)O.x, (_Float16)O.y, (_Float16)O.z, (_Float16)O.w};
-                *reinterpret_cast<h4*>(a->out + (row0 + h) * kHeadDim + d0) = hv;
-                if (d0 == 0) a->lse[row0 + h] = sm.lse[h];
-            } else {
-                const int ps = a->part_stride;
-                const size_t e = ps > 0 ? (row0 + h) * (size_t)ps + slot : (size_t)slot * G + h;
-                *reinterpret_cast<float4*>(a->part_o + e * kHeadDim + d0) = O;
-                if (d0 == 0) a->part_lse[e] = sm.lse[h];
-            }
-        }
-        __syncthreads();   // sm is reused by the next pass or segment
-    }
-}
-
-// One workgroup of 4 waves (one per SIMD) per CU walks its list of segments. Wave i takes pages
-// i, i+4, ... of each segment; its pages of all segments form one stream, each segment's share
-// padded to a multiple of the ring depth NBUF so that a page's ring slot is fixed at compile
-// time. The ring runs across segment boundaries: the next segment's first pages are in flight
-// while a segment is flushed. Partials are written with plain stores and merged by a second
-// kernel, so no workgroup waits for another.
-// COMPACT (the fused cascade step at G = 8, so that a CU holds it beside a prefix workgroup):
-// the flush passes 4 heads at a time, and q rows are staged for at most kStepSegMax segments (the
-// planner caps such a plan's segments per workgroup).
-template <class C, bool COMPACT = false>
-struct BalShared {
-    static constexpr int HP = COMPACT && C::G > 4 ? 4 : C::G;        // heads per flush pass
-    static constexpr int SEGS = COMPACT ? kStepSegMax : kSegMax;      // segments with staged q rows
-    BalSmem<C::G, C::NW * C::RPI, HP> sm;
-    int pg[kRangeMax];                             // the workgroup's page ids
-    u32x4 qs[SEGS][C::G * kHeadDim / 8];           // q rows of each segment
-    int sd[kBalDescInts];                          // descriptor block: header, then segments
-};
-
-// The segments staged in S.sd (nseg of them, at most S's SEGS; page ids of a page-range plan
-// already in S.pg): their q rows and, for other plans, their page ids (positions from the
-// descriptors, in kv_indices of the argument block) are loaded in one round trip, then every
-// wave streams its pages of all segments through one ring, flushing each segment at its end.
-// All threads of the workgroup call it.
-template <class C, bool COMPACT, bool RANGES>
-__device__ __forceinline__ void run_segments(const BalArgs& a, BalShared<C, COMPACT>& S, int nseg,
-                                             bool qpre = false) {
-    constexpr int G = C::G, NW = C::NW, NT = C::NT, NBUF = C::NBUF, LPR = C::LPR;
-    auto& sm = S.sm;
-    int* pg = S.pg;
-    auto& qs = S.qs;
-    int* sd = S.sd;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane / LPR, c = lane % LPR;
-    int* seg = sd + 8;
-    auto fld = [&](int si, int f) { return __builtin_amdgcn_readfirstlane(seg[si * kSegInts + f]); };
-    constexpr int PMAX = kRangeMax / NT, QPS = G * kHeadDim / 8;
-    constexpr int QMAX = (BalShared<C, COMPACT>::SEGS * QPS + NT - 1) / NT;
-    const uint32_t page_bytes = (uint32_t)(kPage * a.Hkv * 256);
-    const uint32_t lbase = (uint32_t)(r * a.Hkv * 256 + c * 16);
-    const uint32_t rstride = (uint32_t)(C::RPI * a.Hkv * 256);
-    auto wcount = [&](int npg) { return npg > wave ? (npg - wave + NW - 1) / NW : 0; };
-
-    // prefetch cursor: segment ps, slot pslot of this wave's (padded) share pcnt / ppad
-    int ps = 0, pslot = 0, pcnt = 0, ppad = 0;
-    auto seek = [&]() {
-        while (ps < nseg) {
-            pcnt = wcount(fld(ps, 3));
-            ppad = (pcnt + NBUF - 1) / NBUF * NBUF;
-            if (ppad > 0) break;
-            ++ps;
-        }
-    };
-    auto issue = [&](PageRegs<C>& buf) {
-        const uint8_t* kb = kargs()->k;
-        const uint8_t* vb = kargs()->v;
-        uint32_t nrec = 0;
-        if (ps < nseg && pslot < pcnt) {
-            const int kvh = fld(ps, 1);
-            const int pid = __builtin_amdgcn_readfirstlane(pg[fld(ps, 2) + wave + NW * pslot]);
-            const size_t off = (size_t)(uint32_t)pid * page_bytes + (size_t)kvh * 256;
-            kb += off;
-            vb += off;
-            nrec = page_bytes - (uint32_t)kvh * 256;
-        }
-        load_page_rsrc<C>(buf, page_rsrc(kb, nrec), page_rsrc(vb, nrec), lbase, rstride);
-        if (ps < nseg && ++pslot == ppad) {
-            ++ps;
-            pslot = 0;
-            seek();
-        }
-    };
-
-    // round trip 2: the q rows of every segment, the page ids of the other plans (item i of the
-    // workgroup's page list is found in the segment whose range [qa, qa + npg) holds it), and for
-    // a page-range plan the first pages of the ring, all issued before any is waited for
-    PageRegs<C> buf[NBUF];
-    {
-        const int npages = fld(nseg - 1, 2) + fld(nseg - 1, 3);
-        const _Float16* qp = kargs()->q;
-        const int32_t* kvi = kargs()->kv_indices;
-        // page-table positions of the page list first (LDS reads only: a search loop with loads
-        // in flight would make the compiler wait for them at every iteration)
-        int src[PMAX];
-        if constexpr (!RANGES) {
-#pragma unroll
-            for (int k = 0; k < PMAX; ++k) {
-                const int i = tid + k * NT;
-                src[k] = -1;
-                if (i < npages) {
-                    int si = 0;
-                    while (si + 1 < nseg && seg[(si + 1) * kSegInts + 2] <= i) ++si;
-                    src[k] = seg[si * kSegInts + 6] + (i - seg[si * kSegInts + 2]);
-                }
-            }
-        }
-        // (every load is issued, past the last segment from segment 0's rows, so that the number
-        // of loads in flight is the same on every path and the waits below stay exact)
-        u32x4 qv4[QMAX];
-        if (!qpre) {
-#pragma unroll
-            for (int k = 0; k < QMAX; ++k) {
-                const int j = tid + k * NT < nseg * QPS ? tid + k * NT : 0;
-                const int si = j / QPS;
-                const size_t row = (size_t)seg[si * kSegInts] * a.Hq + (size_t)seg[si * kSegInts + 1] * G;
-                qv4[k] = reinterpret_cast<const u32x4*>(qp + row * kHeadDim)[j % QPS];
-            }
-        }
+    // (unconditional within the list, so one round trip; none at all for a workgroup whose items
+    // hold no page, whose kv_indices may be empty)
+    if (npages > 0) {
         int pv[PMAX];
-        if constexpr (!RANGES) {
-            // (unconditional within the list, so one round trip; none at all for a workgroup whose
-            // items hold no page, whose kv_indices may be empty)
-            if (npages > 0) {
 #pragma unroll
-                for (int k = 0; k < PMAX; ++k) pv[k] = kvi[max(src[k], 0)];
-            }
-        } else {
-            seek();
-#pragma unroll
-            for (int u = 0; u < NBUF - 1; ++u) issue(buf[u]);
-        }
-        // keeps the stores below after the loads above: the q rows are waited for while the
-        // first pages are still in flight
-        asm volatile("" ::: "memory");
-        if (!qpre) {
-#pragma unroll
-            for (int k = 0; k < QMAX; ++k)
-                if (tid + k * NT < nseg * QPS) qs[(tid + k * NT) / QPS][(tid + k * NT) % QPS] = qv4[k];
-        }
-        if constexpr (!RANGES) {
-#pragma unroll
-            for (int k = 0; k < PMAX; ++k)
-                if (tid + k * NT < npages) pg[tid + k * NT] = pv[k];
-        }
-    }
-    __syncthreads();
-    PD_STAMP(2);
-    if constexpr (!RANGES) {
-        seek();
-#pragma unroll
-        for (int u = 0; u < NBUF - 1; ++u) issue(buf[u]);
-    }
-
-    WaveState<C> st;
-    reset_state<C>(st);
-    for (int si = 0; si < nseg; ++si) {
-        const int npg = fld(si, 3), t0 = fld(si, 4), t1 = fld(si, 5);
-        const int tbase = t0 & ~(kPage - 1);   // first token of the segment's first page
-        f16x2 qv[G][C::PPL][4];
-#pragma unroll
-        for (int h = 0; h < G; ++h)
-#pragma unroll
-            for (int kk = 0; kk < C::PPL; ++kk) {
-                const u32x4 raw = qs[qpre ? 0 : si][h * (kHeadDim / 8) + kk * LPR + c];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) qv[h][kk][e] = as_h2(raw[e]);
-            }
-        const int cnt = wcount(npg);
-        for (int blk = 0; blk < cnt; blk += NBUF) {
-#pragma unroll
-            for (int u = 0; u < NBUF; ++u) {
-                issue(buf[(u + NBUF - 1) % NBUF]);
-                if (blk + u < cnt)
-                    page_step<C>(st, buf[u], qv, tbase + (wave + NW * (blk + u)) * kPage, r, t0, t1,
-                                 a.scale_log2);
-            }
-            if (si == 0 && blk == 0) PD_STAMP(3);
-        }
-        if (si < 12) PD_STAMP(4 + 2 * si);
-        flush_segment<C, BalShared<C, COMPACT>::HP>(sm, st, kargs(),
-                                                    (size_t)fld(si, 0) * a.Hq + (size_t)fld(si, 1) * G,
-                                                    fld(si, 7));
-        reset_state<C>(st);
-        if (si < 12) PD_STAMP(5 + 2 * si);
-    }
-    PD_STAMP(31);
-}
-
-
-// ---- the paired decode: two kv heads per workgroup, pages staged in LDS --------------------
-// A 4-wave workgroup runs two workgroups of a page-range plan, w = 2 x and 2 x + 1: kv heads
-// 2k and 2k + 1 over the same pages. Waves 0-1 serve the first head and waves 2-3 the second,
-// each pair of waves as a plan workgroup of two waves (C::NW = 2), wave i of a head taking pages
-// i, i + 2, ... of every segment. Reading the two heads' rows of a page together (1 KB of every
-// 2 KB token row at once) streams faster than one head's 256-byte rows. The page ring goes
-// through LDS instead of VGPRs: each wave moves its pages with 16-byte buffer loads straight
-// into its own LDS slots (buffer_load ... lds; lane l's pieces land at 16 l of each 1 KB, and
-// lane l reads the same bytes back), two slots per wave. The compiler makes a workgroup barrier
-// wait for every LDS-bound load in flight, so no barrier is placed while pages are in flight
-// except the flushes': q rows go straight to registers (each lane its own pieces), one segment
-// ahead, instead of through LDS.
-template <class C>
-struct PairShared {
-    static constexpr int SLOT = C::RG * C::PPL * 1024 * 2;   // one page of one head: K then V
-    BalSmem<C::G, C::NW * C::RPI> sm[2];           // flush scratch of each head's waves
-    int sd[2][kBalDescInts];                       // the two heads' descriptor blocks
-    int pg[kRangeMax];                             // the range's page ids (the same for both heads)
-    __attribute__((aligned(16))) uint8_t ring[2 * C::NW][2][SLOT];
-};
-
-typedef __attribute__((address_space(3))) void lds_void;
-
-// One page of one head into a wave's LDS slot: lane l's pieces of row group i at
-// slot + (i PPL + kk) * 1024 + 16 l, K then V. Same offsets, resources and cache policy as the
-// VGPR ring's loads (a padding slot's zero-size resources make no memory access).
-template <class C>
-__device__ __forceinline__ void dma_page(uint8_t* slot, __amdgpu_buffer_rsrc_t rk, __amdgpu_buffer_rsrc_t rv,
-                                         uint32_t lbase, uint32_t rstride) {
-    constexpr int HALF = C::RG * C::PPL * 1024;
-#pragma unroll
-    for (int i = 0; i < C::RG; ++i)
-#pragma unroll
-        for (int kk = 0; kk < C::PPL; ++kk) {
-            const int off = (int)(lbase + i * rstride + kk * (C::LPR * 16));
-            uint8_t* d = slot + (i * C::PPL + kk) * 1024;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_void*)d, 16, off, 0, 0, 2);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_void*)(d + HALF), 16, off, 0, 0, 2);
-        }
-}
-template <class C>
-__device__ __forceinline__ void lds_page(PageRegs<C>& pr, const uint8_t* slot, int lane) {
-    constexpr int HALF = C::RG * C::PPL * 1024;
-#pragma unroll
-    for (int i = 0; i < C::RG; ++i)
-#pragma unroll
-        for (int kk = 0; kk < C::PPL; ++kk) {
-            const uint8_t* d = slot + (i * C::PPL + kk) * 1024 + 16 * lane;
-            pr.k[i][kk] = *reinterpret_cast<const u32x4*>(d);
-            pr.v[i][kk] = *reinterpret_cast<const u32x4*>(d + HALF);
-        }
-}
-
-// s_waitcnt vmcnt(N) alone (expcnt and lgkmcnt at their maximum: no wait on them).
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 0xF) | ((N >> 4) << 14));
-}
-// s_waitcnt lgkmcnt(0) alone.
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-
-// Workgroup x of the paired decode (page-range plans only; the plan's Hkv is even). Both heads'
-// descriptor blocks are staged; everything that decides the control flow (segments, pages,
-// tokens) is read from the first, so both halves reach every barrier together. The second head's
-// block contributes its partial slots.
-template <class C>
-__device__ __forceinline__ void pair_body(const BalArgs& a, PairShared<C>& P, int x) {
-    constexpr int G = C::G, NW = C::NW, NT2 = 2 * C::NT, LPR = C::LPR, PPL = C::PPL;
-    constexpr int PMAX = kRangeMax / NT2;
-    constexpr int DPER = (2 * kBalDescInts + NT2 - 1) / NT2;
-    constexpr int OPS = 2 * C::RG * C::PPL;       // buffer loads per page
-    static_assert(C::NBUF == 2, "two LDS slots and two register sets per wave");
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int half = wave / NW, lw = wave % NW, ltid = tid - half * C::NT;
-    const int r = lane / LPR, c = lane % LPR;
-    int* sd0 = P.sd[0];
-    int* seg0 = sd0 + 8;
-    auto fld = [&](int si, int f) { return __builtin_amdgcn_readfirstlane(seg0[si * kSegInts + f]); };
-    PD_STAMP(0);
-    // round trip 1: both descriptor blocks and the range's page ids
-    const int w0 = 2 * x;
-    const int64_t g = w0 / a.Hkv, nnz = kargs()->nnz, ng = kargs()->ngroups;
-    const int64_t lo = nnz * g / ng, hi = nnz * (g + 1) / ng;
-    {
-        const int32_t* desc = kargs()->desc + (size_t)w0 * kBalDescInts;
-        const int32_t* kvi = kargs()->kv_indices + lo;
-        int dv[DPER], pv[PMAX];
-#pragma unroll
-        for (int k = 0; k < DPER; ++k) {
-            const int i = tid + k * NT2;
-            dv[k] = i < 2 * kBalDescInts ? desc[i] : 0;
-        }
-        const int npr = (int)(hi - lo);
-#pragma unroll
-        for (int k = 0; k < PMAX; ++k) {
-            const int i = tid + k * NT2;
-            pv[k] = i < npr ? kvi[i] : 0;
-        }
-#pragma unroll
-        for (int k = 0; k < DPER; ++k) {
-            const int i = tid + k * NT2;
-            if (i < 2 * kBalDescInts) P.sd[i / kBalDescInts][i % kBalDescInts] = dv[k];
-        }
+        for (int k = 0; k < PMAX; ++k) pv[k] = kvi[max(src[k], 0)];
 #pragma unroll
         for (int k = 0; k < PMAX; ++k)
-            if (tid + k * NT2 < npr) P.pg[tid + k * NT2] = pv[k];
+            if (tid + k * NT < npages) S.pg[tid + k * NT] = pv[k];
     }
     __syncthreads();
-    PD_STAMP(1);
-    // (uniform: every thread leaves) either block foreign or empty, or the blocks disagree
-    const int nseg = __builtin_amdgcn_readfirstlane(sd0[0]);
-    const int kvh0 = __builtin_amdgcn_readfirstlane(nseg > 0 ? seg0[1] : 0);
-    if (nseg <= 0 || nseg > kSegMax || nseg != __builtin_amdgcn_readfirstlane(P.sd[1][0]) ||
-        __builtin_amdgcn_readfirstlane(sd0[1]) != kargs()->tag ||
-        __builtin_amdgcn_readfirstlane(P.sd[1][1]) != kargs()->tag || kvh0 < 0 || kvh0 + 1 >= a.Hkv)
-        return;
-    const int kvh = kvh0 + half;
+}
 
-    const uint32_t page_bytes = (uint32_t)(kPage * a.Hkv * 256);
-    const uint32_t lbase = (uint32_t)(r * a.Hkv * 256 + c * 16);
-    const uint32_t rstride = (uint32_t)(C::RPI * a.Hkv * 256);
-    auto wcount = [&](int npg) { return npg > lw ? (npg - lw + NW - 1) / NW : 0; };
-    int ps = 0, pslot = 0, pcnt = 0, ppad = 0;
-    auto seek = [&]() {
-        while (ps < nseg) {
-            pcnt = wcount(fld(ps, 3));
-            ppad = (pcnt + 1) / 2 * 2;
-            if (ppad > 0) break;
-            ++ps;
-        }
+// The segments staged in S.sd (nseg of them, one block per kv head) with their page ids in S.pg:
+// every wave streams its pages of all segments, two pages at a time, flushing each segment at its
+// end. A kv head's WPH waves take every WPH-th page of a segment each. The next block's loads, the
+// next segment's first block included, are in flight while a block is computed or a segment
+// flushed. All threads of the workgroup call it. qpre: the q rows are already in qn.
+template <class C, int LAY>
+__device__ __forceinline__ void run_segments(const BalArgs& a, DecShared<C, LAY>& S, int nseg,
+                                             pf16x8 (&qn)[4], bool qpre = false) {
+    typedef DecShared<C, LAY> Sh;
+    constexpr int G = C::G, WPH = C::WPH, NS = Sh::NS;
+    int* pg = S.pg;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int hh = wave / WPH, lw = wave % WPH;
+    const int l16 = lane & 15, lg = lane >> 4;
+    // this head's segments: one window for the segment being computed, one for the loads' cursor
+    SegWin cur, nxt;
+    cur.init(S.sd[hh] + 8);
+    auto wcount = [&](int npg) { return npg > lw ? (npg - lw + WPH - 1) / WPH : 0; };
+    // this lane's q pieces of segment si: head (l16 & 7) % G, dims 32 ks + 8 lg ..
+    auto qload = [&](int si) {
+        const _Float16* qp = a.q + ((size_t)cur.get(si, 0) * a.Hq + (size_t)cur.get(si, 1) * G + (l16 & 7) % G) * kHeadDim;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) qn[ks] = *reinterpret_cast<const pf16x8*>(qp + 32 * ks + 8 * lg);
     };
-    // stream page k of this wave (padding included) goes to LDS slot k % 2 and register set k % 2
-    int nissued = 0;
-    auto issue = [&]() {
-        const uint8_t* kb = kargs()->k;
-        const uint8_t* vb = kargs()->v;
-        uint32_t nrec = 0;
-        if (ps < nseg && pslot < pcnt) {
-            const int pid = __builtin_amdgcn_readfirstlane(P.pg[fld(ps, 2) + lw + NW * pslot]);
-            const size_t off = (size_t)(uint32_t)pid * page_bytes + (size_t)kvh * 256;
-            kb += off;
-            vb += off;
-            nrec = page_bytes - (uint32_t)kvh * 256;
-        }
-        dma_page<C>(P.ring[wave][nissued & 1], page_rsrc(kb, nrec), page_rsrc(vb, nrec), lbase, rstride);
-        ++nissued;
-        if (ps < nseg && ++pslot == ppad) {
+    if (NS == 1 && !qpre) qload(0);
+
+    // The cursor of the loads: blocks in stream order. advance() leaves the next block's page ids,
+    // head and page count (0 at the end) in scalar registers, read from LDS while the block before
+    // is computed, so that issue() follows the operand reads at once.
+    const uint32_t page_bytes = (uint32_t)(kPage * a.Hkv * 256);
+    nxt = cur;
+    int ps = 0, pslot = 0, pcnt = wcount(nxt.get(0, 3));
+    int have = 0, pid0 = 0, pid1 = 0, pkvh = 0, pb = 0;
+    auto advance = [&]() {
+        while (ps < nseg && pslot >= pcnt) {
             ++ps;
             pslot = 0;
-            seek();
+            pcnt = ps < nseg ? wcount(nxt.get(ps, 3)) : 0;
+        }
+        have = ps < nseg ? min(2, pcnt - pslot) : 0;
+        if (have > 0) {
+            const int qa = nxt.get(ps, 2) + lw + WPH * pslot;
+            const int pv = pg[(lane & 1) && have > 1 ? qa + WPH : qa];
+            pid0 = __builtin_amdgcn_readlane(pv, 0);
+            pid1 = __builtin_amdgcn_readlane(pv, 1);
+            pkvh = nxt.get(ps, 1);
+            pb = nxt.get(ps, 0);
+            pslot += 2;
         }
     };
-    // this lane's q pieces of segment si (head h, piece kk: dims (kk LPR + c) 8 .. + 7)
-    auto qload = [&](int si, u32x4 (&q)[G][PPL]) {
-        const _Float16* qp = kargs()->q + ((size_t)fld(si, 0) * a.Hq + (size_t)kvh * G) * kHeadDim;
+    // Row n = 4 i + lane / 16 of a page, LDS position p = lane % 16 of it: chunk p ^ n of K, p ^ ((n & 7)
+    // << 1) of V (the swizzles that dec_read_block reads).
+    uint32_t koff[4], voff[4];
 #pragma unroll
-        for (int h = 0; h < G; ++h)
+    for (int i = 0; i < 4; ++i) {
+        const int n = 4 * i + lg;
+        koff[i] = (uint32_t)(n * a.Hkv * 256 + ((l16 ^ n) << 4));
+        voff[i] = (uint32_t)(n * a.Hkv * 256 + ((l16 ^ ((n & 7) << 1)) << 4));
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)S.slot[wave][0];
+    // (NS = 2) this lane's 16 bytes of a block's q rows, LDS position lane of them: row r = (lane / 16) % G
+    const uint32_t qoff = (uint32_t)((lg % G) * 256 + (((l16 >> 2 ^ (lg % G)) << 2 | (l16 & 3)) << 4));
+    int sl = 0, nfl = 0;   // the slot of the next block, computed and loaded; loads of the newest block
+    const uint8_t* const kc = a.k;
+    const uint8_t* const vc = a.v;
+    auto issue = [&]() {
+        nfl = 0;
+        if (have <= 0) return;
+        nfl = 8 * have + 1;
+        const uint32_t lds = lds0 + (uint32_t)(sl * Sh::SLOT);
+        if constexpr (NS > 1)
+            dec_dma_q(a.q + ((size_t)pb * a.Hq + (size_t)pkvh * G) * kHeadDim, qoff, lds + kDecSlotBytes);
+        {
+            const size_t off = (size_t)(uint32_t)pid0 * page_bytes + (size_t)pkvh * 256;
 #pragma unroll
-            for (int kk = 0; kk < PPL; ++kk)
-                q[h][kk] = *reinterpret_cast<const u32x4*>(qp + h * kHeadDim + (kk * LPR + c) * 8);
+            for (int i = 0; i < 4; ++i) dec_dma(kc + off, koff[i], lds + 1024 * i);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dec_dma(vc + off, voff[i], lds + 2 * kDecPageBytes + 1024 * i);
+        }
+        if (have > 1) {
+            const size_t off = (size_t)(uint32_t)pid1 * page_bytes + (size_t)pkvh * 256;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dec_dma(kc + off, koff[i], lds + kDecPageBytes + 1024 * i);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dec_dma(vc + off, voff[i], lds + 3 * kDecPageBytes + 1024 * i);
+        }
     };
 
-    // round trip 2: the first segment's q pieces, then the first two pages of the ring
-    u32x4 qn[G][PPL];
-    qload(0, qn);
-    seek();
-    issue();
-    issue();
-    wait_vm<OPS>();            // page 0 (page 1 in flight)
-    PageRegs<C> pr[2];
-    lds_page<C>(pr[0], P.ring[wave][0], lane);
     PD_STAMP(2);
-
-    WaveState<C> st;
-    reset_state<C>(st);
+    advance();
+    issue();
+    advance();
+    if constexpr (NS > 1) {
+        sl = 1;
+        issue();
+        advance();
+        sl = 0;
+    }
+    const bool is_lo = (l16 & 8) != 0;
+    const float lo_a = is_lo ? kLoScale : 1.f, lo_b = is_lo ? -kLoScale : 0.f;
+    DecState st;
+    int par = 0;
     for (int si = 0; si < nseg; ++si) {
-        const int npg = fld(si, 3), t0 = fld(si, 4), t1 = fld(si, 5);
-        const int tbase = t0 & ~(kPage - 1);
-        f16x2 qv[G][PPL][4];
+        const int npg = cur.get(si, 3), t0 = cur.get(si, 4), t1 = cur.get(si, 5);
+        const int b_ = cur.get(si, 0), kvh = cur.get(si, 1), ps_ = cur.get(si, 7);
+        const int tbase = t0 & ~(kPage - 1);   // first token of the segment's first page
+        pf16x8 q[4];
+        if constexpr (NS == 1) {
 #pragma unroll
-        for (int h = 0; h < G; ++h)
-#pragma unroll
-            for (int kk = 0; kk < PPL; ++kk)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) qv[h][kk][e] = as_h2(qn[h][kk][e]);
-        if (si + 1 < nseg) qload(si + 1, qn);   // (waited for at the next segment)
+            for (int ks = 0; ks < 4; ++ks) q[ks] = qn[ks];
+            if (si + 1 < nseg && !qpre) qload(si + 1);   // (a one-sequence plan has one segment's rows)
+        }
+        dec_reset(st);
         const int cnt = wcount(npg);
         for (int blk = 0; blk < cnt; blk += 2) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                // page k (parity u) is in pr[u]; its slot is refilled with page k + 2 once the
-                // reads of it are done; page k + 1 (in flight since the last step) is waited for
-                // and read into pr[u ^ 1] while page k is computed
-                wait_lgkm0();
-                issue();
-                wait_vm<OPS>();
-                lds_page<C>(pr[u ^ 1], P.ring[wave][u ^ 1], lane);
-                if (blk + u < cnt)
-                    page_step<C>(st, pr[u], qv, tbase + (lw + NW * (blk + u)) * kPage, r, t0, t1,
-                                 a.scale_log2);
+            DecBlock b;
+            if constexpr (NS > 1) {
+                dec_wait_loads(nfl);
+                dec_read_q<G>(q, S.slot[wave][sl] + kDecSlotBytes, l16, lg);
+            } else {
+                dec_wait_loads();
             }
+            dec_read_block(b, S.slot[wave][sl], l16, lg);
+            dec_wait_lds();
+            issue();
+            advance();
+            if (NS > 1) sl ^= 1;
+            const int tok0 = tbase + (lw + WPH * blk) * kPage;
+            dec_block(st, b, q, tok0, blk + 1 < cnt ? tok0 + WPH * kPage : t1, t0, t1, a.scale_log2, lo_a, lo_b, lg);
             if (si == 0 && blk == 0) PD_STAMP(3);
         }
         if (si < 12) PD_STAMP(4 + 2 * si);
-        // this head's slot: its own block's field (the two blocks differ only in head and slot)
-        const int slot = __builtin_amdgcn_readfirstlane(P.sd[half][8 + si * kSegInts + 7]);
-        flush_segment<C, G>(P.sm[half], st, kargs(), (size_t)fld(si, 0) * a.Hq + (size_t)kvh * G, slot, ltid);
-        reset_state<C>(st);
+        dec_flush<C, LAY>(S, st, par, kargs(), (size_t)b_ * a.Hq + (size_t)kvh * G, ps_);
+        par ^= 1;
         if (si < 12) PD_STAMP(5 + 2 * si);
     }
     PD_STAMP(31);
 }
 
-// The body of one balanced-decode workgroup w (the kernel's argument block must start with the
-// BalArgs `a`, which kargs() reads).
-template <class C, bool UNI = false, bool COMPACT = false, bool RANGES = false>
-__device__ __forceinline__ void balanced_body(const BalArgs& a, BalShared<C, COMPACT>& S, int w,
+// The body of one balanced-decode workgroup: workgroups HP w .. HP w + HP - 1 of the plan (HP > 1:
+// neighbouring kv heads of one page range). The kernel's argument block must start with the
+// BalArgs `a`, which kargs() reads.
+template <class C, bool UNI = false, int LAY = kLayWide, bool RANGES = false>
+__device__ __forceinline__ void balanced_body(const BalArgs& a, DecShared<C, LAY>& S, int x,
                                               const UniArgs* u = nullptr) {
     static_assert(!(UNI && RANGES), "the uniform split builds its own descriptors");
-    constexpr int G = C::G, NT = C::NT;
+    static_assert(C::HP == 1 || RANGES || UNI, "several heads share a page list");
+    constexpr int G = C::G, NT = C::NT, HP = C::HP, PMAX = DecShared<C, LAY>::PGMAX / NT;
     int* pg = S.pg;
-    auto& qs = S.qs;
-    int* sd = S.sd;
-    const int tid = threadIdx.x;
+    int* sd = S.sd[0];
+    const int tid = threadIdx.x, w = x * HP;
     // Segment fields are staged in LDS (sd: a header of 8 ints, then the segments) and read back
-    // wave-uniform by run_segments: global (vector) loads of them would count against the same
-    // wait counter as the ring's page loads, and a non-uniform value in a buffer resource would
-    // turn every page load into a loop over lanes.
+    // wave-uniform by run_segments.
     int* seg = sd + 8;
-    // timestamps (timeline build only): 0 start, 1 descriptors (and page ids) staged, 2 q rows
-    // staged, 3 the first ring step computed, 4 + 2 s / 5 + 2 s segment s streamed / flushed
+    // timestamps (timeline build only): 0 start, 1 descriptors (and page ids) staged, 2 the first
+    // loads issued next, 3 the first block computed, 4 + 2 s / 5 + 2 s segment s streamed / flushed
     // (s < 12), 31 done; thread 0 of the workgroup
     PD_STAMP(0);
-    constexpr int PMAX = kRangeMax / NT, QPS = G * kHeadDim / 8;
-    // A page-range plan (RANGES: ngroups > 0) gives workgroup w = g * Hkv + kvh the pages
-    // [lo, hi) of the page table (relative to kv_indptr[0]), lo = nnz g / ngroups: its page list is
-    // known from the kernel arguments, so the page ids are loaded together with the descriptor
-    // block, and the ring's first pages together with the q rows.
-    int64_t lo = 0, hi = 0;
-    bool qpre = false;   // q rows staged in round trip 1 (a one-sequence page-range plan)
-    if constexpr (RANGES) {
-        const int64_t g = w / a.Hkv, nnz = kargs()->nnz, ng = kargs()->ngroups;
-        lo = nnz * g / ng;
-        hi = nnz * (g + 1) / ng;
-        qpre = kargs()->qrow_b >= 0;
-    }
+    pf16x8 qn[4];
+    bool qpre = false;   // q rows loaded in round trip 1 (a one-sequence page-range plan)
     int nseg;
     if constexpr (!UNI) {
-        // round trip 1: the whole descriptor block (one int per thread), and the page ids of a
-        // page-range plan
-        const int32_t* desc = kargs()->desc + (size_t)w * kBalDescInts;
-        const int32_t* kvi = kargs()->kv_indices + lo;   // (pointers read from the arguments once)
-        const int dv = tid < kBalDescInts ? desc[tid] : 0;
-        int pv[PMAX];
-        const int npr = (int)(hi - lo);
-#pragma unroll
-        for (int k = 0; k < PMAX; ++k) {
-            const int i = tid + k * NT;
-            pv[k] = i < npr ? kvi[i] : 0;
-        }
-        // a one-sequence plan: the q rows of (qrow_b, this workgroup's kv head) in the same trip
-        // (every segment uses them), so that round trip 2 carries only the ring's first pages
-        u32x4 qv = {0u, 0u, 0u, 0u};
+        // A page-range plan (RANGES: ngroups > 0) gives workgroup w = g * Hkv + kvh the pages
+        // [lo, hi) of the page table (relative to kv_indptr[0]), lo = nnz g / ngroups: its page list
+        // is known from the kernel arguments, so the page ids are loaded together with the
+        // descriptor block(s), in round trip 1.
+        uint32_t g = 0, lo = 0, npr = 0;
         if constexpr (RANGES) {
-            if (qpre) {
-                const size_t row = (size_t)kargs()->qrow_b * a.Hq + (size_t)(w % a.Hkv) * G;
-                if (tid < QPS) qv = reinterpret_cast<const u32x4*>(kargs()->q + row * kHeadDim)[tid];
-            }
+            g = dec_div((uint32_t)w, (uint32_t)a.Hkv, a.hkv_m);
+            lo = dec_range(a, g);
+            npr = min(dec_range(a, g + 1) - lo, (uint32_t)DecShared<C, LAY>::PGMAX);
+            qpre = DecShared<C, LAY>::NS == 1 && a.qrow_b >= 0;
         }
-        if (tid < kBalDescInts) sd[tid] = dv;
+        const int dst = a.desc_stride;   // <= kBalDescInts <= NT
+        const int32_t* desc = a.desc + (size_t)w * dst;
+        const int32_t* kvi = a.kv_indices + lo;
+        int dv[HP], pv[PMAX];
 #pragma unroll
-        for (int k = 0; k < PMAX; ++k)
-            if (tid + k * NT < npr) pg[tid + k * NT] = pv[k];
-        if (qpre && tid < QPS) qs[0][tid] = qv;
+        for (int h = 0; h < HP; ++h) dv[h] = desc[h * dst + min(tid, dst - 1)];
+        if constexpr (RANGES) {
+            // (NG <= nnz: every range holds a page)
+            pv[0] = kvi[min((uint32_t)tid, npr - 1)];
+            // a one-sequence plan: the q rows of (qrow_b, this wave's kv head) in the same trip
+            // (every segment uses them)
+            if (qpre) {
+                const int lane = tid & 63, hh = __builtin_amdgcn_readfirstlane(tid >> 6) / C::WPH;
+                const _Float16* qp = a.q + ((size_t)a.qrow_b * a.Hq + (size_t)(w - g * a.Hkv + hh) * G +
+                                            (lane & 7) % G) * kHeadDim + 8 * (lane >> 4);
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks) qn[ks] = *reinterpret_cast<const pf16x8*>(qp + 32 * ks);
+            }
+            if (npr > NT) {   // (wave-uniform)
+#pragma unroll
+                for (int k = 1; k < PMAX; ++k) pv[k] = kvi[min((uint32_t)(tid + k * NT), npr - 1)];
+#pragma unroll
+                for (int k = 1; k < PMAX; ++k) pg[tid + k * NT] = pv[k];
+            }
+            pg[tid] = pv[0];
+        }
+#pragma unroll
+        for (int h = 0; h < HP; ++h)
+            if (tid < dst) S.sd[h][tid] = dv[h];
         __syncthreads();
         PD_STAMP(1);
         nseg = __builtin_amdgcn_readfirstlane(sd[0]);
-        // (uniform: every thread leaves) no segment, or not this plan's descriptor block: the
+        // (uniform: every thread leaves) no segment, or not this plan's descriptor block(s): the
         // workspace was written over since the upload, and nothing here is to be trusted
-        if (nseg <= 0 || nseg > BalShared<C, COMPACT>::SEGS ||
-            __builtin_amdgcn_readfirstlane(sd[1]) != kargs()->tag)
-            return;
+        if (nseg <= 0 || nseg > kSegMax) return;
+#pragma unroll
+        for (int h = 0; h < HP; ++h)
+            if (__builtin_amdgcn_readfirstlane(S.sd[h][0]) != nseg ||
+                __builtin_amdgcn_readfirstlane(S.sd[h][1]) != a.tag)
+                return;
     } else {
-        // items w, w + W, ...: thread t builds the descriptor of the t-th (the decode_partial
-        // rule, 01_decode_attention.cu:88-97: keys [kv_start + chunk * chunk_tokens, + chunk_tokens)
-        // clipped to the sequence; an empty range writes 0 / -inf). t0 is the first key of the
-        // range, which need not start a page: keys are numbered from its page's first token.
-        nseg = min(u->per_wg, (u->n_items - w + a.W - 1) / a.W);
+        // items x, x + W, ... (W workgroups): thread t builds the descriptors of the t-th, one per
+        // head (the decode_partial rule, 01_decode_attention.cu:88-97: keys [kv_start + chunk *
+        // chunk_tokens, + chunk_tokens) clipped to the sequence; an empty range writes 0 / -inf). t0
+        // is the first key of the range, which need not start a page: keys are numbered from its
+        // page's first token.
+        nseg = min(u->per_wg, (u->n_items - x + a.W - 1) / a.W);
         if (nseg <= 0) return;   // uniform: the host sizes the grid so that every workgroup has items
         if (tid < nseg) {
-            const int item = w + tid * a.W;
+            const int item = x + tid * a.W, groups = a.Hkv / HP;
             const int pair = item / u->num_chunks, chunk = item - pair * u->num_chunks;
-            const int b = pair / a.Hkv, kvh = pair - b * a.Hkv;
+            const int b = pair / groups, kvh = (pair - b * groups) * HP;
             const int pb = u->kv_indptr[b], np = u->kv_indptr[b + 1] - pb;
             // (a last-page length outside [1, 16] is clamped: no key past the sequence's pages)
             const int len = np > 0 ? (np - 1) * kPage + min(kPage, max(1, u->kv_last[b])) : 0;
             const int kbeg = u->kv_start + chunk * u->chunk_tokens;
             const int kend = max(kbeg, min(len, kbeg + u->chunk_tokens));
             const int pf = kbeg / kPage;
-            int* sg = seg + tid * kSegInts;
-            sg[0] = b;
-            sg[1] = kvh;
-            sg[3] = kend > kbeg ? (kend - 1) / kPage - pf + 1 : 0;
-            sg[4] = kbeg;
-            sg[5] = kend;
-            sg[6] = pb + pf;
-            sg[7] = a.out != nullptr ? -1 : u->chunk_base + chunk;
+#pragma unroll
+            for (int h = 0; h < HP; ++h) {
+                int* sg = S.sd[h] + 8 + tid * kSegInts;
+                sg[0] = b;
+                sg[1] = kvh + h;
+                sg[3] = kend > kbeg ? (kend - 1) / kPage - pf + 1 : 0;
+                sg[4] = kbeg;
+                sg[5] = kend;
+                sg[6] = pb + pf;
+                sg[7] = a.out != nullptr ? -1 : u->chunk_base + chunk;
+            }
         }
         __syncthreads();
         // page-list offsets: exclusive prefix sum of the page counts
         if (tid < nseg) {
             int qa = 0;
             for (int j = 0; j < tid; ++j) qa += seg[j * kSegInts + 3];
-            seg[tid * kSegInts + 2] = qa;
+#pragma unroll
+            for (int h = 0; h < HP; ++h) S.sd[h][8 + tid * kSegInts + 2] = qa;
         }
         __syncthreads();
         PD_STAMP(1);
     }
 
-    run_segments<C, COMPACT, RANGES>(a, S, nseg, qpre);
+    if constexpr (!RANGES) stage_pages<C, LAY>(a, S, nseg);
+    run_segments<C, LAY>(a, S, nseg, qn, qpre);
 }
 
 // ---- page ranges found on the device (the drop-in decode_attention without a host plan) -----
-template <class C, bool COMPACT>
+template <class C>
 struct DevShared {
-    BalShared<C, COMPACT> b;
+    DecShared<C, kLayOne> b;
     int ip[kDevMaxB + 1];      // kv_indptr
+    int piece[kDevMaxB];       // the sequences with a piece in the range, in order
+    int pb[kDevMaxB];          // of those: attended pages before the sequence, its attended pages,
+    int cnt[kDevMaxB];         // its length (indexed by sequence; written where they are needed)
+    int len[kDevMaxB];
     int wx[2 * C::NW];         // per-wave piece counts and clip flags of the common-case guess
-    int sc[C::NW + 1];         // block-scan scratch; sc[NW]: the current batch's first page
+    int sc[C::NW];             // block-scan scratch
+    int keep[4];               // the range, the end of the keys and the workgroup, for later batches
 };
 
 // Exclusive prefix sum of v over the workgroup's threads, in thread order, and the total. All
@@ -1330,16 +964,17 @@ __device__ __forceinline__ int block_exscan(int v, int* sc, int& total) {
 // page ids are contiguous in kv_indices: that case is assumed at once, its page ids are loaded
 // while one barrier settles whether it holds, and its pieces run as a host page-range plan's do.
 // Otherwise two block scans give the prefix sums of the attended pages and the index of each
-// sequence piece in the range, and the pieces run in batches of at most SEGS segments (a range of
+// sequence piece in the range, and the pieces run in batches of at most kSegMax segments (a range of
 // many short sequences), each batch like a host plan's workgroup (run_segments).
-template <class C, bool COMPACT>
-__device__ __forceinline__ void dev_body(const DevArgs& da, DevShared<C, COMPACT>& D, int w) {
-    constexpr int G = C::G, NW = C::NW, NT = C::NT, SEGS = BalShared<C, COMPACT>::SEGS;
+template <class C>
+__device__ __forceinline__ void dev_body(const DevArgs& da, DevShared<C>& D, int wg) {
+    constexpr int G = C::G, HP = C::HP, NW = C::NW, NT = C::NT, SEGS = kSegMax;
     constexpr int PMAX = kRangeMax / NT;
     static_assert(4 * NT >= kDevMaxB + 1, "four sequences per thread");
     const BalArgs& a = da.d;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, B = a.B, Hkv = a.Hkv;
-    const int g = w / Hkv, kvh = w - g * Hkv;
+    // (w: the slots' workgroup index of the first of this workgroup's HP kv heads)
+    const int w = wg * HP, g = w / Hkv;
     const int64_t NG = a.ngroups;
     PD_STAMP(0);
     // (unconditional loads at clamped indices, B >= 1: a conditional load per element would be
@@ -1441,75 +1076,82 @@ __device__ __forceinline__ void dev_body(const DevArgs& da, DevShared<C, COMPACT
         }
         f0 = block_exscan<NW>(nf, D.sc, ntot);
     }
-    if (w == 0) {
+    if (wg == 0) {
 #pragma unroll
         for (int k = 0; k < 4; ++k)
             if (4 * tid + k <= B) da.prefix[4 * tid + k] = pb[k];
     }
     if (lo == hi) {
         // an empty range (fewer pages than ranges): its slots are read as empty by the merge
-        if (tid < 2 * G) a.part_lse[((size_t)2 * w + tid / G) * G + tid % G] = -INFINITY;
+        if (tid < 2 * HP * G) a.part_lse[(size_t)2 * w * G + tid] = -INFINITY;
         return;
     }
-    int* sd = D.b.sd;
-    int* seg = sd + 8;
-    // Descriptors of segments [sb, sb + nseg) whose page list starts at page bs0 of the attended
-    // pages; the caller publishes them with a barrier.
-    auto describe = [&](int sb, int nseg, int bs0) {
+    // The piece of sequence b (attended pages [p, p + c), length len) as segment si of a batch whose
+    // page list starts at attended page bs0.
+    auto describe = [&](int si, int b, int p, int c, int len, int bs0, int lo, int hi, int ks, int ke, int w) {
+        const int s0 = max(p, lo), s1 = min(p + c, hi), kvh = w % a.Hkv;
+        const int pa0 = ks / kPage + (s0 - p), pa1 = ks / kPage + (s1 - p);
+#pragma unroll
+        for (int h = 0; h < HP; ++h) {
+            int* sg = D.b.sd[h] + 8 + si * kSegInts;
+            sg[0] = b;
+            sg[1] = kvh + h;
+            sg[2] = s0 - bs0;
+            sg[3] = s1 - s0;
+            sg[4] = max(ks, pa0 * kPage);
+            sg[5] = min(min(len, ke), pa1 * kPage);
+            sg[6] = D.ip[b] + pa0;
+            sg[7] = (s0 == p && s1 == p + c) ? -1 : (s0 == lo && p < lo) ? 2 * (w + h) : 2 * (w + h) + 1;
+        }
+    };
+    // Batches of at most SEGS segments. The common case is one batch, whose page list is the range's
+    // pages, already loaded. The first batch is described from the registers above, the others from
+    // LDS, so that none of that state stays live through the page loops.
+    const bool one = fast && ntot <= SEGS;
+    int nseg = min(SEGS, ntot);
+    {
         int fi = f0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             if (!fl[k]) continue;
-            const int si = fi++ - sb;
-            if (si < 0 || si >= nseg) continue;
-            const int b = 4 * tid + k;
-            const int s0 = max(pb[k], lo), s1 = min(pb[k] + cnt[k], hi);
-            const int pa0 = ks / kPage + (s0 - pb[k]), pa1 = ks / kPage + (s1 - pb[k]);
-            const int kend = min(lenv[k], ke);
-            int* sg = seg + si * kSegInts;
-            sg[0] = b;
-            sg[1] = kvh;
-            sg[2] = s0 - bs0;
-            sg[3] = s1 - s0;
-            sg[4] = max(ks, pa0 * kPage);
-            sg[5] = min(kend, pa1 * kPage);
-            sg[6] = D.ip[b] + pa0;
-            sg[7] = (s0 == pb[k] && s1 == pb[k] + cnt[k]) ? -1
-                    : (s0 == lo && pb[k] < lo) ? 2 * w : 2 * w + 1;
+            const int b = 4 * tid + k, si = fi++;
+            if (si < SEGS) describe(si, b, pb[k], cnt[k], lenv[k], lo, lo, hi, ks, ke, w);
+            if (ntot > SEGS) {
+                D.piece[si] = b;
+                D.pb[b] = pb[k];
+                D.cnt[b] = cnt[k];
+                D.len[b] = lenv[k];
+            }
         }
-        if (tid == 0) sd[0] = nseg;
-    };
-    // The common case, every piece of the range in one batch: the range's page list is its pages,
-    // and the segment runner is the last thing the workgroup does, so none of the state above stays
-    // live through its page loop (which then compiles to the plan path's schedule: measured 7%
-    // slower streaming otherwise).
-    if (fast && ntot <= SEGS) {
-        describe(0, ntot, lo);
+    }
+    if (one) {
 #pragma unroll
         for (int k = 0; k < PMAX; ++k)
             if (tid + k * NT < hi - lo) D.b.pg[tid + k * NT] = pv[k];
-        __syncthreads();
-        PD_STAMP(30);
-        run_segments<C, COMPACT, true>(a, D.b, ntot);
-        return;
     }
-    // Batches: each one's page list starts at its first segment's first page in the range.
-    for (int sb = 0; sb < ntot; sb += SEGS) {
-        const int nseg = min(SEGS, ntot - sb);
-        {
-            int fi = f0;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (fl[k]) {
-                    if (fi == sb) D.sc[NW] = max(pb[k], lo);
-                    ++fi;
-                }
+    if (tid == 0) {
+        D.keep[0] = lo;
+        D.keep[1] = hi;
+        D.keep[2] = ke;
+        D.keep[3] = w;
+    }
+    __syncthreads();
+    PD_STAMP(30);
+    pf16x8 qn[4];
+    for (int sb = 0;;) {
+        if (!one) stage_pages<C, kLayOne>(a, D.b, nseg);
+        run_segments<C, kLayOne>(a, D.b, nseg, qn);
+        sb += SEGS;
+        if (sb >= ntot) break;
+        nseg = min(SEGS, ntot - sb);
+        const int bs0 = D.pb[D.piece[sb]];   // (a later batch starts with a whole sequence or its start)
+        __syncthreads();
+        if (tid < nseg) {
+            const int b = D.piece[sb + tid];
+            describe(tid, b, D.pb[b], D.cnt[b], D.len[b], bs0, D.keep[0], D.keep[1], da.kv_start, D.keep[2],
+                     D.keep[3]);
         }
         __syncthreads();
-        const int bs0 = D.sc[NW];
-        describe(sb, nseg, bs0);
-        __syncthreads();
-        run_segments<C, COMPACT, false>(a, D.b, nseg);
     }
 }
 
@@ -1538,38 +1180,27 @@ __global__ __launch_bounds__(kMergeThreads) void merge_ranges_kernel(DevMergeArg
     merge_store(st, a.out + (size_t)row * kHeadDim, a.lse + row);
 }
 
-// At G = 8 the per-page VALU work is about twice G = 4's and no longer hides under the page's
-// memory time with one wave per SIMD, so the kernel uses the compact LDS layout (61 KB) and the
-// planner gives it two workgroups per CU: the two waves on each SIMD overlap one's arithmetic with
-// the other's loads.
+// One kv head per workgroup (C::HP = 1), or HP neighbouring heads of a page-range plan: workgroup x
+// runs the plan's workgroups HP x .. HP x + HP - 1.
 template <class C, bool RANGES>
-__global__ __launch_bounds__(C::NT) void decode_balanced_kernel(BalArgs a) {
-    __shared__ BalShared<C, (C::G > 4)> S;
-    balanced_body<C, false, (C::G > 4), RANGES>(a, S, blockIdx.x);
-}
-
-// The paired decode (two kv heads per 4-wave workgroup, pages staged in LDS): workgroup x runs
-// the page-range plan's workgroups 2 x and 2 x + 1.
-template <class C>
-__global__ __launch_bounds__(2 * C::NT) void decode_pair_kernel(BalArgs a) {
-    __shared__ PairShared<C> S;
-    pair_body<C>(a, S, blockIdx.x);
+__global__ __launch_bounds__(C::NT, 2) void decode_balanced_kernel(BalArgs a) {
+    __shared__ DecShared<C, kLayWide> S;
+    balanced_body<C, false, kLayWide, RANGES>(a, S, blockIdx.x);
 }
 
 // The reference-shaped uniform split on the balanced body (items of equal key ranges, descriptors
 // built in the kernel from the device page table).
 template <class C>
-__global__ __launch_bounds__(C::NT) void decode_uniform_kernel(UniArgs u) {
-    __shared__ BalShared<C, (C::G > 4)> S;   // G = 8: compact, two workgroups per CU (as above)
-    balanced_body<C, true, (C::G > 4)>(u.d, S, blockIdx.x, &u);
+__global__ __launch_bounds__(C::NT, 2) void decode_uniform_kernel(UniArgs u) {
+    __shared__ DecShared<C, kLayWide> S;
+    balanced_body<C, true>(u.d, S, blockIdx.x, &u);
 }
 
-// The drop-in decode_attention over page ranges found on the device (G = 8: the compact layout,
-// two workgroups per CU, as for the plan path).
+// The drop-in decode_attention over page ranges found on the device.
 template <class C>
-__global__ __launch_bounds__(C::NT) void decode_ranges_kernel(DevArgs d) {
-    __shared__ DevShared<C, (C::G > 4)> S;
-    dev_body<C, (C::G > 4)>(d, S, blockIdx.x);
+__global__ __launch_bounds__(C::NT, 2) void decode_ranges_kernel(DevArgs d) {
+    __shared__ DevShared<C> S;
+    dev_body<C>(d, S, blockIdx.x);
 }
 
 // The fused cascade step: blocks [0, n_dec) are the suffix decode's workgroups, the rest the
@@ -1581,12 +1212,12 @@ __global__ __launch_bounds__(C::NT) void decode_ranges_kernel(DevArgs d) {
 template <class C, bool RANGES>
 __global__ __launch_bounds__(C::NT, 2) void cascade_step_kernel(StepArgs s) {
     static_assert(C::NT == kPrefixThreads, "both roles use the same workgroup shape");
-    typedef BalShared<C, (C::G > 4)> Dec;   // G = 8: the compact layout (fits beside a prefix workgroup)
+    typedef DecShared<C, kLayStep> Dec;
     constexpr size_t SB = sizeof(Dec) > sizeof(PSmem) ? sizeof(Dec) : sizeof(PSmem);
-    __shared__ __align__(16) unsigned char raw[SB];
+    __shared__ __align__(256) unsigned char raw[SB];
     const int i = blockIdx.x;
     if (i < s.n_dec) {
-        balanced_body<C, false, (C::G > 4), RANGES>(s.d, *reinterpret_cast<Dec*>(raw), i);
+        balanced_body<C, false, kLayStep, RANGES>(s.d, *reinterpret_cast<Dec*>(raw), i);
     } else {
         const int j = i - s.n_dec, n_items = s.p.num_chunks;
         prefix_workgroup(s.p, *reinterpret_cast<PSmem*>(raw), j % n_items, 0, j / n_items);
@@ -1606,18 +1237,12 @@ int occupancy_of(const void* fn, int threads) {
 // split: 64x1K 57.0 vs 64.3 us, 1x32K 39.9 vs 39.8 us, 8x8K 57.2 vs 57.8 us.
 template <int G>
 using PartialCfg = Cfg<G, 16, 4, 2>;
-// Balanced body (plan/run, the uniform split and the cascade's suffix): 4 waves (one per SIMD,
-// one workgroup per CU), 16 lanes per row (four row groups per wave, so the end-of-segment merge
-// is two permlane steps), a two-page ring: one page in flight while the other is computed. Deeper
-// rings measured slower at every shape (4 pages: 30.6 vs 28.5 us back to back at 1x32K, 46.1 vs
-// 44.9 us at 64x1K; at G = 8, 3 pages: 29.3 vs 28.6 us and 42.8 vs 41.4 us): more bytes in
-// flight only lengthen the memory queues.
+// MFMA body (plan/run, the uniform split, device ranges and the cascade's suffix): one kv head per
+// 4-wave workgroup, or two neighbouring heads of a page range, two waves each.
 template <int G>
-using BalCfg = Cfg<G, 16, 4, 2>;
-// Paired decode: each kv head's half of the workgroup is two waves (the workgroup is still four
-// waves, one per SIMD), a two-page ring per wave in LDS.
+using BalCfg = DecCfg<G, 1>;
 template <int G>
-using PairCfg = Cfg<G, 16, 2, 2>;
+using PairCfg = DecCfg<G, 2>;
 
 template <class C>
 void launch_p(const PartialArgs& a, hipStream_t s) {
@@ -1630,7 +1255,7 @@ void launch_b(const BalArgs& a, hipStream_t s) {
 }
 template <class C>
 void launch_pair(const BalArgs& a, hipStream_t s) {
-    decode_pair_kernel<C><<<a.W / 2, 2 * C::NT, 0, s>>>(a);
+    decode_balanced_kernel<C, true><<<a.W / C::HP, C::NT, 0, s>>>(a);
 }
 template <class C>
 void launch_u(const UniArgs& a, hipStream_t s) {
@@ -1638,8 +1263,12 @@ void launch_u(const UniArgs& a, hipStream_t s) {
 }
 template <class C>
 void launch_step(const StepArgs& a, hipStream_t s) {
-    if (a.d.ngroups > 0) cascade_step_kernel<C, true><<<a.n_dec + a.n_pre, C::NT, 0, s>>>(a);
-    else cascade_step_kernel<C, false><<<a.n_dec + a.n_pre, C::NT, 0, s>>>(a);
+    if constexpr (C::HP == 1)
+        if (a.d.ngroups <= 0) {
+            cascade_step_kernel<C, false><<<a.n_dec + a.n_pre, C::NT, 0, s>>>(a);
+            return;
+        }
+    cascade_step_kernel<C, true><<<a.n_dec + a.n_pre, C::NT, 0, s>>>(a);
 }
 template <class C>
 void launch_r(const DevArgs& a, hipStream_t s) {
@@ -1690,25 +1319,27 @@ hipError_t launch_decode_balanced(const BalArgs& a, int G, hipStream_t s) {
 }
 
 hipError_t launch_decode_pair(const BalArgs& a, int G, hipStream_t s) {
-    if (G != 1 && G != 2 && G != 4) return hipErrorInvalidValue;
+    if (G != 1 && G != 2 && G != 4 && G != 8) return hipErrorInvalidValue;
     if (a.ngroups <= 0 || a.Hkv % 2 != 0 || a.W % 2 != 0 || a.W <= 0) return hipErrorInvalidValue;
-    if (G == 1) launch_pair<PairCfg<1>>(a, s);
-    else if (G == 2) launch_pair<PairCfg<2>>(a, s);
-    else launch_pair<PairCfg<4>>(a, s);
+    PD_DISPATCH(PairCfg, G, launch_pair, a, s);
     return hipGetLastError();
 }
 
-hipError_t launch_decode_uniform(const UniArgs& a, int G, hipStream_t s) {
+hipError_t launch_decode_uniform(const UniArgs& a, int G, int hp, hipStream_t s) {
     if (G != 1 && G != 2 && G != 4 && G != 8) return hipErrorInvalidValue;
+    if (hp != 1 && (hp != 2 || a.d.Hkv % 2 != 0)) return hipErrorInvalidValue;
     if (a.d.W <= 0) return hipSuccess;
-    PD_DISPATCH(BalCfg, G, launch_u, a, s);
+    if (hp == 2) PD_DISPATCH(PairCfg, G, launch_u, a, s);
+    else PD_DISPATCH(BalCfg, G, launch_u, a, s);
     return hipGetLastError();
 }
 
-hipError_t launch_cascade_step(const StepArgs& a, int G, hipStream_t s) {
+hipError_t launch_cascade_step(const StepArgs& a, int G, int hp, hipStream_t s) {
     if (G != 1 && G != 2 && G != 4 && G != 8) return hipErrorInvalidValue;
+    if (hp != 1 && (hp != 2 || a.d.Hkv % 2 != 0 || a.d.ngroups <= 0)) return hipErrorInvalidValue;
     if (a.n_dec + a.n_pre <= 0) return hipSuccess;
-    PD_DISPATCH(BalCfg, G, launch_step, a, s);
+    if (hp == 2) PD_DISPATCH(PairCfg, G, launch_step, a, s);
+    else PD_DISPATCH(BalCfg, G, launch_step, a, s);
     return hipGetLastError();
 }
 
@@ -1721,10 +1352,12 @@ hipError_t launch_merge_split(const MergeArgs& a, int n_entries, hipStream_t s) 
     return hipGetLastError();
 }
 
-hipError_t launch_decode_ranges(const DevArgs& a, int G, hipStream_t s) {
+hipError_t launch_decode_ranges(const DevArgs& a, int G, int hp, hipStream_t s) {
     if (G != 1 && G != 2 && G != 4 && G != 8) return hipErrorInvalidValue;
+    if (hp != 1 && (hp != 2 || a.d.Hkv % 2 != 0)) return hipErrorInvalidValue;
     if (a.d.W <= 0) return hipSuccess;
-    PD_DISPATCH(BalCfg, G, launch_r, a, s);
+    if (hp == 2) PD_DISPATCH(PairCfg, G, launch_r, a, s);
+    else PD_DISPATCH(BalCfg, G, launch_r, a, s);
     return hipGetLastError();
 }
 

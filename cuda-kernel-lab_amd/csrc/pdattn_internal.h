@@ -34,7 +34,7 @@ struct PartialArgs {
 // Balanced decode: the host planner gives each workgroup a range of pages of one kv head -- by
 // default range g of the page sequence cut into W / Hkv equal ranges for workgroup g * Hkv + h,
 // kv head h; or the units [U w / W, U (w+1) / W) of the pairs' chunks, kv head fastest -- cut into
-// segments (one per sequence or chunk piece), described in desc[w * kBalDescInts ..]:
+// segments (one per sequence or chunk piece), described in desc[w * desc_stride ..]:
 //   desc[0] = number of segments; desc[1] = the plan's tag (a launch whose tag argument differs
 //   finds someone else's bytes there and does nothing); segment s at desc[8 + kSegInts * s] =
 //   {b, kvh, qa, npg, t0, t1, jpos, slot}: sequence b, kv head kvh, pages [qa, qa + npg) of the
@@ -42,10 +42,10 @@ struct PartialArgs {
 //   page-table position jpos of its first page (relative to kv_indptr[0]), and the partial slot
 //   it writes (-1: the segment is the whole pair and writes the final out / lse).
 constexpr int kSegMax = 24;                // segments per workgroup
-constexpr int kStepSegMax = 8;             // segments per workgroup of the fused cascade step at G = 8
 constexpr int kSegInts = 8;
 constexpr int kBalDescInts = 8 + kSegMax * kSegInts;
 constexpr int kRangeMax = 2048;            // pages per workgroup (page ids staged in LDS)
+constexpr int kStepRangeMax = 1024;        // of them in the fused cascade step's decode role
 
 struct BalArgs {
     const _Float16* q;
@@ -54,7 +54,7 @@ struct BalArgs {
     const int32_t*  kv_indices;   // offset by kv_indptr[0]
     _Float16*       out;
     float*          lse;
-    const int32_t*  desc;         // [W * kBalDescInts]
+    const int32_t*  desc;         // [W * desc_stride]
     float*          part_o;       // [slots * G * 128] partial outputs (normalized)
     float*          part_lse;     // [slots * G]
     int B, Hq, Hkv, W;
@@ -71,6 +71,10 @@ struct BalArgs {
     // >= 0 (page-range plans of one sequence): every segment of every workgroup is of sequence
     // qrow_b, so a workgroup's q rows (kv head w % Hkv) are loaded with its descriptor block
     int qrow_b = -1;
+    int desc_stride = 0;          // ints per descriptor block (header and the most segments of a block)
+    // ranges and kv heads of a page-range plan without a division: nnz / ngroups, nnz % ngroups, and
+    // floor((2^32 - 1) / d) for d = ngroups and d = Hkv
+    uint32_t range_q = 0, range_r = 0, range_m = 0, hkv_m = 0;
 };
 
 // The reference-shaped uniform split (decode_partial / decode_attention) run by the balanced
@@ -187,16 +191,16 @@ hipError_t launch_decode_partial(const PartialArgs& a, int G, hipStream_t s);
 hipError_t launch_merge_states(const float* part_o, const float* part_lse, _Float16* out,
                                float* lse, int rows, int num_chunks, hipStream_t s);
 hipError_t launch_decode_balanced(const BalArgs& a, int G, hipStream_t s);
-// The paired variant of a page-range plan (two kv heads per workgroup, W / 2 workgroups; G in
-// 1, 2, 4 and Hkv even).
+// A page-range plan run two kv heads per workgroup (W / 2 workgroups; Hkv even). hp below: kv heads
+// per workgroup (1, or 2 where Hkv is even).
 hipError_t launch_decode_pair(const BalArgs& a, int G, hipStream_t s);
-hipError_t launch_decode_uniform(const UniArgs& a, int G, hipStream_t s);
+hipError_t launch_decode_uniform(const UniArgs& a, int G, int hp, hipStream_t s);
 hipError_t launch_merge_split(const MergeArgs& a, int n_entries, hipStream_t s);
-hipError_t launch_decode_ranges(const DevArgs& a, int G, hipStream_t s);
+hipError_t launch_decode_ranges(const DevArgs& a, int G, int hp, hipStream_t s);
 hipError_t launch_merge_ranges(const DevMergeArgs& a, hipStream_t s);
 hipError_t launch_fill_i32(int32_t* p, int32_t value, size_t n, hipStream_t s);
 hipError_t launch_cascade_prefix(const PrefixArgs& a, int G, hipStream_t s);
-hipError_t launch_cascade_step(const StepArgs& a, int G, hipStream_t s);
+hipError_t launch_cascade_step(const StepArgs& a, int G, int hp, hipStream_t s);
 hipError_t launch_append_kv(const AppendArgs& a, int cus, hipStream_t s);
 hipError_t launch_stream_read(const void* buf, size_t bytes, uint32_t* sink, int grid, hipStream_t s);
 hipError_t launch_flush(void* buf, size_t bytes, int grid, hipStream_t s);

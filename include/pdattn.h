@@ -194,17 +194,16 @@ typedef struct pdattn_plan_info {
     int     segments;          /* segments over all workgroups                            */
     int     merge_entries;     /* pairs merged by the second launch (0: single launch)    */
     int     schedule_ints;     /* int32 count of pdattn_plan_get_schedule's output        */
-    int     paired;            /* 1: the decode launch runs workgroups w and w + 1 (kv heads
-                                  2k, 2k + 1 of one page range) as one workgroup of the paired
-                                  kernel, W / 2 workgroups                                 */
+    int     paired;            /* 1: a G <= 4 plan of two workgroups per CU (w and w + 1, kv heads
+                                  2k, 2k + 1 of one page range, run as one kernel workgroup)
+                                  that splits no sequence over workgroups; 0 for every other
+                                  plan, also where kernel workgroups hold two heads          */
 } pdattn_plan_info;
 
 /* Build a plan from host copies of kv_indptr [B+1] and kv_last_page_len [B]. force_workgroups > 0
- * overrides the grid size (one workgroup per CU by default, two at G = 8; it grows when a
- * workgroup would exceed its segment or page limits). At G <= 4 with an even Hkv the default is
- * first planned with two workgroups per CU for the paired kernel, which runs workgroups w and
- * w + 1 (kv heads 2k, 2k + 1 of one page range) as one, its pages staged in LDS; if that plan
- * splits any sequence over workgroups, one workgroup per CU is planned instead (info.paired).
+ * overrides the grid size (by default one workgroup per CU, or two where Hkv is even and the batch
+ * has 8 pages per range or more sequences than ranges: the kernel then runs workgroups w and w + 1, kv heads 2k and 2k + 1 of one
+ * page range, as one; it grows when a workgroup would exceed its segment or page limits).
  * chunk_pages > 0, or a grid that is not a
  * multiple of Hkv, selects the other partition: chunks of up to chunk_pages pages (64 by default)
  * of one (sequence, kv head) pair, ordered sequence-major, then by chunk position, kv head
@@ -288,8 +287,7 @@ typedef struct pdattn_cascade_plan pdattn_cascade_plan;
 /* How pdattn_cascade_decode runs the prefix pass and the suffix decode (pdattn_cascade_set_mode).
  * FUSED: one launch whose first workgroups decode the suffix and whose others run the prefix
  * items; both roles are 4-wave workgroups small enough for a CU to hold one of each, so every CU
- * streams suffix pages while its matrix core works on the prefix; the default (at G = 8 the
- * decode role uses a compact LDS layout so that it fits). SERIAL: the prefix launch, then the
+ * streams suffix pages while its matrix core works on the prefix; the default. SERIAL: the prefix launch, then the
  * suffix decode (the reference's order, cascade_decode 01_decode_attention.cu:703-712). TWO_STREAMS:
  * the prefix launch forked onto a second stream owned by the plan, joined before the merge. All
  * three compute the same partials with the same kernels' arithmetic: the results are bitwise
