@@ -421,7 +421,6 @@ __device__ __forceinline__ KArgPtr kargs() {
 // deterministic. keepA(k), evaluated after the loads, drops source k of A (a slot the decode launch
 // did not write). The state is left in every lane: merged output acc / ws, lse m + ln ws.
 constexpr int kMergeThreads = 256;
-constexpr int kMergeU = 4;   // sources of a list per lane per round trip
 struct MState {
     float m, ws;
     float4 acc;
@@ -449,19 +448,29 @@ __device__ __forceinline__ void mstate_fold_dpp(MState& s) {
     s.m = M;
 }
 
-__device__ __forceinline__ int merge_d0() { return 32 * (int)(threadIdx.x >> 6) + 4 * (int)((threadIdx.x & 63) >> 3); }
+// The first of this lane's 4 dims. A row is one workgroup of 4 waves (32 dims each), or (WIDE) four
+// workgroups of one wave, blockIdx % 4 being the wave's place: few rows with many sources each then
+// spread over four times as many CUs.
+template <bool WIDE>
+__device__ __forceinline__ int merge_d0() {
+    const int w = WIDE ? (int)(blockIdx.x & 3) : (int)(threadIdx.x >> 6);
+    return 32 * w + 4 * (int)((threadIdx.x & 63) >> 3);
+}
+template <bool WIDE>
+__device__ __forceinline__ int merge_row() { return WIDE ? (int)(blockIdx.x >> 2) : (int)blockIdx.x; }
 
 // The sources of a row are list A then list B, as one list of A.n + B.n: source k is A's k-th
 // for k < A.n, else B's (k - A.n)-th. Lane r of each 8-lane group takes sources k0 + r + 8 u
-// (u < kMergeU), loaded unconditionally: a lane past the last source reloads the last one, and
+// (u < U), loaded unconditionally: a lane past the last source reloads the last one, and
 // the list a source comes from is a per-lane select of its address, so every lane issues the same
 // loads and no load waits for another (conditional loads would make the compiler copy the
-// results, and wait for them, where the branches join). 8 kMergeU sources per round trip.
-__device__ __forceinline__ void merge_load(const MSrc& A, const MSrc& B, int k0, float (&l)[kMergeU],
-                                           float4 (&o)[kMergeU]) {
-    const int r = threadIdx.x & 7, d0 = merge_d0(), n = A.n + B.n;
+// results, and wait for them, where the branches join). 8 U sources per round trip.
+template <int U>
+__device__ __forceinline__ void merge_load(const MSrc& A, const MSrc& B, int k0, int d0, float (&l)[U],
+                                           float4 (&o)[U]) {
+    const int r = threadIdx.x & 7, n = A.n + B.n;
 #pragma unroll
-    for (int u = 0; u < kMergeU; ++u) {
+    for (int u = 0; u < U; ++u) {
         const int k = min(k0 + r + 8 * u, n - 1);
         const bool inA = k < A.n;
         const size_t i = inA ? (size_t)k * A.stride : (size_t)(k - A.n) * B.stride;
@@ -478,13 +487,12 @@ __device__ __forceinline__ void merge_load(const MSrc& A, const MSrc& B, int k0,
 // by exp(m - max(m, l)) (exactly 1 when l <= m) and the source (lse l, normalized output o) added
 // with weight exp(l - max(m, l)); an empty source (l = -inf) weighs 0. keepA(k) drops sources of
 // list A (B's are all kept).
-template <class KeepA>
+template <int U, class KeepA>
 __device__ __forceinline__ void merge_fold(MState& s, const MSrc& A, const MSrc& B, int k0,
-                                           const float (&l)[kMergeU], const float4 (&o)[kMergeU],
-                                           KeepA keepA) {
+                                           const float (&l)[U], const float4 (&o)[U], KeepA keepA) {
     const int r = threadIdx.x & 7, n = A.n + B.n;
 #pragma unroll
-    for (int u = 0; u < kMergeU; ++u) {
+    for (int u = 0; u < U; ++u) {
         const int k = k0 + r + 8 * u;
         const bool ok = k < n && (k >= A.n || keepA(k)) && l[u] != -INFINITY;
         const float lv = ok ? l[u] : -INFINITY;
@@ -501,20 +509,20 @@ __device__ __forceinline__ void merge_fold(MState& s, const MSrc& A, const MSrc&
     }
 }
 
-template <class KeepA>
-__device__ __forceinline__ MState merge_lanes(const MSrc& A, const MSrc& B, KeepA keepA) {
-    constexpr int SPT = 8 * kMergeU;   // sources per round trip
+template <int U, class KeepA>
+__device__ __forceinline__ MState merge_lanes(const MSrc& A, const MSrc& B, int d0, KeepA keepA) {
+    constexpr int SPT = 8 * U;   // sources per round trip
     MState s{-INFINITY, 0.f, make_float4(0.f, 0.f, 0.f, 0.f)};
     const int n = A.n + B.n;
     if (n > 0) {
-        float l[kMergeU];
-        float4 o[kMergeU];
-        merge_load(A, B, 0, l, o);
+        float l[U];
+        float4 o[U];
+        merge_load<U>(A, B, 0, d0, l, o);
         __builtin_amdgcn_sched_barrier(0);   // every load above is issued before anything waits
-        merge_fold(s, A, B, 0, l, o, keepA);
+        merge_fold<U>(s, A, B, 0, l, o, keepA);
         for (int k0 = SPT; k0 < n; k0 += SPT) {
-            merge_load(A, B, k0, l, o);
-            merge_fold(s, A, B, k0, l, o, keepA);
+            merge_load<U>(A, B, k0, d0, l, o);
+            merge_fold<U>(s, A, B, k0, l, o, keepA);
         }
     }
     mstate_fold_dpp<0xB1>(s);    // quad_perm [1,0,3,2]
@@ -525,9 +533,8 @@ __device__ __forceinline__ MState merge_lanes(const MSrc& A, const MSrc& B, Keep
 
 // Writes a merged row: lane 0 of each 8-lane group its 4 fp16 outputs, the first of them the lse.
 // A row whose every source is empty gets out = 0, lse = -inf.
-__device__ __forceinline__ void merge_store(const MState& s, _Float16* out_row, float* lse_out) {
+__device__ __forceinline__ void merge_store(const MState& s, int d0, _Float16* out_row, float* lse_out) {
     if ((threadIdx.x & 7) != 0) return;
-    const int d0 = merge_d0();
     const float inv = s.ws > 0.f ? 1.f / s.ws : 0.f;
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
     const h4 hv = {(_Float16)(s.acc.x * inv), (_Float16)(s.acc.y * inv), (_Float16)(s.acc.z * inv),
@@ -570,16 +577,18 @@ __global__ __launch_bounds__(C::NT) void decode_partial_kernel(PartialArgs a) {
 
 // ---- log-sum-exp merge: the reference's merge_states launch shape -------------------------
 // One workgroup per row, `num_chunks` consecutive partial slots.
+template <int U, bool WIDE>
 __global__ __launch_bounds__(kMergeThreads) void merge_states_kernel(const float* __restrict__ part_o,
                                                                       const float* __restrict__ part_lse,
                                                                       _Float16* __restrict__ out,
                                                                       float* __restrict__ lse_out,
                                                                       int num_chunks) {
-    const size_t row = blockIdx.x;
+    const size_t row = merge_row<WIDE>();
+    const int d0 = merge_d0<WIDE>();
     const MSrc A{part_lse + row * num_chunks, part_o + row * num_chunks * kHeadDim, 1, num_chunks};
     const MSrc B{part_lse, part_o, 1, 0};
-    const MState st = merge_lanes(A, B, [](int) { return true; });
-    merge_store(st, out + row * kHeadDim, lse_out + row);
+    const MState st = merge_lanes<U>(A, B, d0, [](int) { return true; });
+    merge_store(st, d0, out + row * kHeadDim, lse_out + row);
 }
 
 // ---- balanced launch -------------------------------------------------------------------------
@@ -591,9 +600,9 @@ __global__ __launch_bounds__(kMergeThreads) void merge_states_kernel(const float
 // in one round trip (the header and entry as vector loads through a zero lane offset the compiler
 // cannot see through, so that they count against the same counter as the partials and nothing is
 // waited for before all are issued). Otherwise the partials follow the entry.
-template <bool RECT>
+template <bool RECT, int U, bool WIDE>
 __global__ __launch_bounds__(kMergeThreads) void merge_split_kernel(MergeArgs a) {
-    const int G = a.G, e = blockIdx.x / G, h = blockIdx.x - e * G;
+    const int G = a.G, er = merge_row<WIDE>(), e = er / G, h = er - e * G, d0 = merge_d0<WIDE>();
     int z = 0;
     asm volatile("v_mov_b32 %0, 0" : "=v"(z));
     // header {tag, n_entries, cmax, 0} and entry {b, kvh, slot0, nc}
@@ -607,7 +616,7 @@ __global__ __launch_bounds__(kMergeThreads) void merge_split_kernel(MergeArgs a)
         const size_t row = (size_t)e * G + h;          // with extra partials entry e is pair e
         const MSrc A{a.part_lse + sl0, a.part_o + sl0 * kHeadDim, (size_t)G, cmax};
         const MSrc B{a.extra_lse + row * n_extra, a.extra_o + row * n_extra * kHeadDim, 1, n_extra};
-        st = merge_lanes(A, B, [&](int k) { return k < en.w; });
+        st = merge_lanes<U>(A, B, d0, [&](int k) { return k < en.w; });
         if (en.w > cmax || (n_extra > 0 && (int64_t)en.x * a.Hkv + en.y != (int64_t)e)) return;
     } else {
         if (hd.x != a.tag || en.z < 0 || en.w < 0 || (int64_t)en.z + en.w > a.n_slots) return;
@@ -616,11 +625,11 @@ __global__ __launch_bounds__(kMergeThreads) void merge_split_kernel(MergeArgs a)
         const size_t row = ((size_t)en.x * a.Hkv + en.y) * G + h;
         const MSrc A{a.part_lse + sl0, a.part_o + sl0 * kHeadDim, (size_t)G, en.w};
         const MSrc B{a.extra_lse + row * n_extra, a.extra_o + row * n_extra * kHeadDim, 1, n_extra};
-        st = merge_lanes(A, B, [](int) { return true; });
+        st = merge_lanes<U>(A, B, d0, [](int) { return true; });
     }
     if (hd.x != a.tag || en.x < 0 || en.x >= a.B || en.y < 0 || en.y >= a.Hkv) return;
     const size_t orow = ((size_t)en.x * a.Hkv + en.y) * G + h;
-    merge_store(st, a.out + orow * kHeadDim, a.lse + orow);
+    merge_store(st, d0, a.out + orow * kHeadDim, a.lse + orow);
 }
 
 // The page list of the segments staged in S.sd, where it is not one range of kv_indices: item i of
@@ -1158,8 +1167,9 @@ __device__ __forceinline__ void dev_body(const DevArgs& da, DevShared<C>& D, int
 // Merge of the sequences split over ranges: one workgroup per row (b, q head); the prefix sums
 // written by the decode launch say which ranges hold sequence b's pages. A row of a sequence
 // with no attended key gets 0 / -inf; a sequence within one range was written by its workgroup.
+template <int U, bool WIDE>
 __global__ __launch_bounds__(kMergeThreads) void merge_ranges_kernel(DevMergeArgs a) {
-    const int row = blockIdx.x, b = row / a.Hq, hq = row - b * a.Hq;
+    const int row = merge_row<WIDE>(), d0 = merge_d0<WIDE>(), b = row / a.Hq, hq = row - b * a.Hq;
     const int kvh = hq / a.G, hh = hq - kvh * a.G;
     const int64_t pb = a.prefix[b], pe = a.prefix[b + 1], N = a.prefix[a.B];
     MState st{-INFINITY, 0.f, make_float4(0.f, 0.f, 0.f, 0.f)};
@@ -1171,13 +1181,13 @@ __global__ __launch_bounds__(kMergeThreads) void merge_ranges_kernel(DevMergeArg
         const size_t i1 = ((size_t)((g0 + 1) * a.Hkv + kvh) * 2) * a.G + hh;     // slot 2 w of g0 + 1
         const MSrc A{a.part_lse + i0, a.part_o + i0 * kHeadDim, 1, 1};
         const MSrc Bs{a.part_lse + i1, a.part_o + i1 * kHeadDim, (size_t)2 * a.Hkv * a.G, (int)(g1 - g0)};
-        st = merge_lanes(A, Bs, [](int) { return true; });
+        st = merge_lanes<U>(A, Bs, d0, [](int) { return true; });
     } else {
         // (the fold leaves the empty state: out 0, lse -inf)
         const MSrc E{a.part_lse, a.part_o, 1, 0};
-        st = merge_lanes(E, E, [](int) { return true; });
+        st = merge_lanes<U>(E, E, d0, [](int) { return true; });
     }
-    merge_store(st, a.out + (size_t)row * kHeadDim, a.lse + row);
+    merge_store(st, d0, a.out + (size_t)row * kHeadDim, a.lse + row);
 }
 
 // One kv head per workgroup (C::HP = 1), or HP neighbouring heads of a page-range plan: workgroup x
@@ -1305,11 +1315,31 @@ hipError_t launch_decode_partial(const PartialArgs& a, int G, hipStream_t s) {
     return hipGetLastError();
 }
 
+// The merge kernels: `n` sources per row (the most, or about as many) choose how many a lane loads in
+// one round trip, so that short lists load nothing twice and long ones take one trip.
+template <class F>
+hipError_t launch_merge(int n, int64_t rows, F launch) {
+    const bool wide = rows <= 64;
+    const dim3 grid((unsigned)(wide ? 4 * rows : rows)), block(wide ? 64 : kMergeThreads);
+    auto go = [&](auto u) {
+        if (wide) launch(u, std::true_type{}, grid, block);
+        else launch(u, std::false_type{}, grid, block);
+    };
+    if (n <= 8) go(std::integral_constant<int, 1>{});
+    else if (n <= 16) go(std::integral_constant<int, 2>{});
+    else if (n <= 24) go(std::integral_constant<int, 3>{});
+    else if (n <= 32) go(std::integral_constant<int, 4>{});
+    else go(std::integral_constant<int, 8>{});
+    return hipGetLastError();
+}
+
 hipError_t launch_merge_states(const float* part_o, const float* part_lse, _Float16* out,
                                float* lse, int rows, int num_chunks, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    merge_states_kernel<<<rows, kMergeThreads, 0, s>>>(part_o, part_lse, out, lse, num_chunks);
-    return hipGetLastError();
+    return launch_merge(num_chunks, rows, [&](auto u, auto wide, dim3 grid, dim3 block) {
+        merge_states_kernel<decltype(u)::value, decltype(wide)::value><<<grid, block, 0, s>>>(part_o, part_lse, out,
+                                                                                              lse, num_chunks);
+    });
 }
 
 hipError_t launch_decode_balanced(const BalArgs& a, int G, hipStream_t s) {
@@ -1347,8 +1377,11 @@ int occupancy_cascade_step(int G) { PD_DISPATCH_RET(BalCfg, G, occ_step); }
 
 hipError_t launch_merge_split(const MergeArgs& a, int n_entries, hipStream_t s) {
     if (n_entries <= 0) return hipSuccess;
-    if (a.cmax > 0) merge_split_kernel<true><<<n_entries * a.G, kMergeThreads, 0, s>>>(a);
-    else merge_split_kernel<false><<<n_entries * a.G, kMergeThreads, 0, s>>>(a);
+    if (a.cmax > 0)
+        return launch_merge(a.cmax + a.n_extra, (int64_t)n_entries * a.G, [&](auto u, auto wide, dim3 grid, dim3 block) {
+            merge_split_kernel<true, decltype(u)::value, decltype(wide)::value><<<grid, block, 0, s>>>(a);
+        });
+    merge_split_kernel<false, 4, false><<<n_entries * a.G, kMergeThreads, 0, s>>>(a);
     return hipGetLastError();
 }
 
@@ -1363,8 +1396,9 @@ hipError_t launch_decode_ranges(const DevArgs& a, int G, int hp, hipStream_t s) 
 
 hipError_t launch_merge_ranges(const DevMergeArgs& a, hipStream_t s) {
     if (a.B <= 0) return hipSuccess;
-    merge_ranges_kernel<<<a.B * a.Hq, kMergeThreads, 0, s>>>(a);
-    return hipGetLastError();
+    return launch_merge(a.ngroups / a.B + 2, (int64_t)a.B * a.Hq, [&](auto u, auto wide, dim3 grid, dim3 block) {
+        merge_ranges_kernel<decltype(u)::value, decltype(wide)::value><<<grid, block, 0, s>>>(a);
+    });
 }
 
 int occupancy_decode_partial(int G) { PD_DISPATCH_RET(PartialCfg, G, occ_p); }
