@@ -784,7 +784,7 @@ def timeline(args):
     cp = pdattn.CascadePlan(base, bt.indptr, bt.indices, bt.lens, t["indices"])
     cws = pdattn.Workspace()
     info = cp.info()
-    nd, npre = info.suffix_workgroups, info.prefix_workgroups
+    npre = info.prefix_workgroups
     for mode in ("cold", "b2b"):
         reset("decode")
         runs = []
@@ -798,6 +798,7 @@ def timeline(args):
                 for _ in range(4):
                     cp.decode(t["out"], t["lse"], cws, s)
             runs.append(grab("decode"))
+        nd = int((runs[0][:, 0] > 0).sum()) - npre   # (the decode role's workgroups come first)
         report("cascade 64x(8192+512) step, decode role", mode, nd, summary(runs, 0, nd, DECODE_STAMPS))
         report("cascade 64x(8192+512) step, prefix role", mode, npre,
                summary(runs, nd, nd + npre, PREFIX_STAMPS))

@@ -14,6 +14,7 @@ import subprocess
 
 HEAD_DIM = 128
 PAGE = 16
+_SCALE = 1.0 / HEAD_DIM ** 0.5
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 _ROOT = os.path.dirname(_PKG_DIR)
@@ -191,17 +192,23 @@ def _check(status: int, where: str):
 
 def ptr(x) -> int | None:
     """Device address of x: an int, None, or an object with data_ptr()."""
-    if x is None:
-        return None
-    if isinstance(x, int):
-        return x
-    return int(x.data_ptr())
+    try:
+        p = x.data_ptr()
+    except AttributeError:
+        if x is None or isinstance(x, int):
+            return x
+        raise
+    return p if p.__class__ is int else int(p)
 
 
 def stream_ptr(s) -> int | None:
-    if s is None or isinstance(s, int):
-        return s
-    return int(s.cuda_stream)
+    try:
+        p = s.cuda_stream
+    except AttributeError:
+        if s is None or isinstance(s, int):
+            return s
+        raise
+    return p if p.__class__ is int else int(p)
 
 
 def host_i32(a):
@@ -316,6 +323,7 @@ class Plan:
     def __init__(self, kv_indptr, kv_last_page_len, B: int, Hq: int, Hkv: int,
                  force_workgroups: int = 0, chunk_pages: int = 0):
         self._h = ctypes.c_void_p()
+        self._run = lib().pdattn_plan_run
         ip, ipp = host_i32(kv_indptr)
         la, lap = host_i32(kv_last_page_len)
         _check(lib().pdattn_plan_create(ipp, lap, B, Hq, Hkv, force_workgroups, chunk_pages,
@@ -356,11 +364,13 @@ class Plan:
 
     def run(self, q, k_cache, v_cache, kv_indptr, kv_indices, kv_last_page_len, out, lse,
             workspace, nbytes: int, sm_scale=None, stream=None):
-        sc = (1.0 / HEAD_DIM ** 0.5) if sm_scale is None else sm_scale
-        _check(lib().pdattn_plan_run(self._h, ptr(q), ptr(k_cache), ptr(v_cache), ptr(kv_indptr),
-                                     ptr(kv_indices), ptr(kv_last_page_len), ctypes.c_float(sc),
-                                     ptr(out), ptr(lse), ptr(workspace), nbytes, stream_ptr(stream)),
-               "pdattn_plan_run")
+        # (a decode step calls this once per layer: the native function is looked up once, and the scale
+        # is converted by the call itself)
+        st = self._run(self._h, ptr(q), ptr(k_cache), ptr(v_cache), ptr(kv_indptr), ptr(kv_indices),
+                       ptr(kv_last_page_len), _SCALE if sm_scale is None else sm_scale, ptr(out), ptr(lse),
+                       ptr(workspace), nbytes, stream_ptr(stream))
+        if st:
+            _check(st, "pdattn_plan_run")
 
     def run_part(self, parts: int, q, k_cache, v_cache, kv_indptr, kv_indices, kv_last_page_len, out,
                  lse, workspace, nbytes: int, sm_scale=None, stream=None):
