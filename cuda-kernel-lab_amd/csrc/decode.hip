@@ -766,8 +766,11 @@ __device__ __forceinline__ void run_segments(const BalArgs& a, DecShared<C, LAY>
         advance();
         sl = 0;
     }
-    const bool is_lo = (l16 & 8) != 0;
-    const float lo_a = is_lo ? kLoScale : 1.f, lo_b = is_lo ? -kLoScale : 0.f;
+    const DecWeights wc = dec_weights(l16);
+    // (a scale of 0 would make a masked key's -inf a NaN: every exponent is then 0 all the same)
+    float scale = a.scale_log2 == 0.f ? 0x1p-126f : a.scale_log2;
+    asm("" : "+v"(scale));
+    const float scale2 = fabsf(scale);
     DecState st;
     int par = 0;
     for (int si = 0; si < nseg; ++si) {
@@ -778,6 +781,7 @@ __device__ __forceinline__ void run_segments(const BalArgs& a, DecShared<C, LAY>
         if constexpr (NS == 1) {
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) q[ks] = qn[ks];
+            dec_sign_q(q, scale);
             if (si + 1 < nseg && !qpre) qload(si + 1);   // (a one-sequence plan has one segment's rows)
         }
         dec_reset(st);
@@ -794,13 +798,16 @@ __device__ __forceinline__ void run_segments(const BalArgs& a, DecShared<C, LAY>
             dec_wait_lds();
             issue();
             advance();
-            if (NS > 1) sl ^= 1;
+            if (NS > 1) {
+                dec_sign_q(q, scale);
+                sl ^= 1;
+            }
             const int tok0 = tbase + (lw + WPH * blk) * kPage;
-            dec_block(st, b, q, tok0, blk + 1 < cnt ? tok0 + WPH * kPage : t1, t0, t1, a.scale_log2, lo_a, lo_b, lg);
+            dec_block(st, b, q, tok0, blk + 1 < cnt ? tok0 + WPH * kPage : t1, t0, t1, scale2, wc, lg);
             if (si == 0 && blk == 0) PD_STAMP(3);
         }
         if (si < 12) PD_STAMP(4 + 2 * si);
-        dec_flush<C, LAY>(S, st, par, kargs(), (size_t)b_ * a.Hq + (size_t)kvh * G, ps_);
+        dec_flush<C, LAY>(S, st, par, kargs(), (size_t)b_ * a.Hq + (size_t)kvh * G, ps_, scale2);
         par ^= 1;
         if (si < 12) PD_STAMP(5 + 2 * si);
     }

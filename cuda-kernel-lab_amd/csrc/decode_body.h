@@ -6,11 +6,17 @@
 //   S^T = K Q^T      v_mfma_f32_16x16x32_f16, A = 16 keys x 32 dims, B = 32 dims x 16 columns
 //   O^T += V^T P^T   A = 16 dims x 32 keys, B = 32 keys x 16 columns
 //
-// A decode batch has only G <= 8 rows per kv head, so half of the 16 columns would idle. They hold
-// the weights' low halves instead: columns 0-7 are the heads with p rounded to fp16, columns 8-15
-// the same heads with (p - fp16(p)) * 2^11 rounded to fp16, and the output is the first plus 2^-11
-// times the second. The PV product then sees every weight to 22 bits (an error of 2^-23 of the
-// weight on average, fp32's own rounding is 2^-25), at no extra MFMA; scores and sums are fp32.
+// The weights p (fp32, at most 1) enter the PV product whole, as three fp16 parts of p * 2^15:
+//   hi = fp16(p 2^15),  mid = fp16((p 2^15 - hi) 2^11),  lo = fp16((p 2^15 - hi) 2^11 - mid)
+// and the output is (hi V + 2^-11 (mid V + lo V)) 2^-15. A decode batch has only G <= 8 rows per kv head,
+// so half of the 16 columns would idle: columns 0-7 (head c % 8 % G) hold hi and columns 8-15 mid; lo
+// goes through a second MFMA into the latter. hi and mid take 11 bits each and lo the rest: the sum is p
+// exactly, all 24 bits, for p >= 2^-27 of the running maximum's weight 1; below that it is within 2^-51
+// (fp16's smallest value, 2^-24, at lo's scale), which no fp16 output can show. Scores, sums and
+// accumulators are fp32. Error of the fp32 partials against 64 bits with fp32 weights on the vector unit
+// / with hi and mid alone, rounded scaled scores / this: 4096 keys 3.4e-7 / 2.7e-7 / 2.6e-7, q eight
+// times larger 6.1e-7 / 5.8e-7 / 5.2e-7, 8192 keys at G = 8 4.5e-7 / 3.4e-7 / 3.4e-7, q eight times larger
+// 6.5e-7 / 6.7e-7 / 5.9e-7.
 //
 // Staging: a wave moves its own pages with 16-byte direct global->LDS loads into its own 16 KB slots
 // (K and V of two pages), so the loop has no workgroup barrier. Per block the wave waits for its
@@ -45,7 +51,8 @@ struct DecCfg {
 constexpr int kDecPageBytes = kPage * kHeadDim * 2;      // one page of one head, K or V
 constexpr int kDecSlotBytes = 4 * kDecPageBytes;         // K of two pages, then V of two pages
 constexpr int kDecQBytes = 4 * kHeadDim * 2;             // q rows of up to 4 heads
-constexpr float kLoScale = 2048.f;                       // scale of the weights' low halves
+constexpr float kWScale = 32768.f;                       // scale of the weights in the PV product
+constexpr float kLoScale = 2048.f;                       // and, on top, of their lower parts
 constexpr float kDecLn2 = 0.69314718055994531f;
 
 // LDS layouts: kLayWide holds two blocks per wave (one at G = 8); kLayOne one block and leaves room for
@@ -101,9 +108,8 @@ struct SegWin {
 };
 static_assert(kSegInts == 8 && kBalDescInts == 8 + 3 * 64, "three windows of 8 segments");
 
-// One wave's running state: column c of the accumulators is head c % 8 (its fp16 weights for
-// c < 8, their low halves for c >= 8). m is the same in the four lanes of a column; l is the sum
-// over the lane's own keys.
+// One wave's running state: the accumulators (times 2^15) of the columns above. m, the largest unscaled
+// score, is the same in the four lanes of a column; l is the sum over the lane's own keys.
 struct DecState {
     float m, l;
     pf32x4 acc[8];
@@ -216,15 +222,44 @@ __device__ __forceinline__ void dec_read_q(pf16x8 (&q)[4], uint8_t* qs, int l16,
                                                (lds_u8*)qs + r * 256 + ((((ks ^ r) << 2) | lg) << 4)));
 }
 
-// One 32-key block: scores, online softmax (base 2, on scores scaled by scale2), PV product. tok0 /
-// tok1: (wave-uniform) token index of the two pages' first slots; keys outside [tb, te) are masked
-// (a padding page: tok1 >= te). A masked key weighs 0 and, since 0 * NaN is not 0, its V elements
-// are zeroed as well: slots the cache never filled may hold any bits. Its K row only feeds its own
-// score, which is replaced.
-// lo_a, lo_b: (1, 0) in columns 0-7, (2^11, -2^11) in columns 8-15: fma(fp16(p), lo_b, p lo_a) is p
-// or its scaled rounding error, both exact.
+// q of a negative sm_scale (wave-uniform) with its signs turned: exact, and the scale is positive from there.
+__device__ __forceinline__ void dec_sign_q(pf16x8 (&q)[4], float scale) {
+    if (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, scale)) >= 0) return;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) q[ks] = __builtin_bit_cast(pf16x8, __builtin_bit_cast(pu32x4, q[ks]) ^ 0x80008000u);
+}
+
+// The constants of the weights' parts, per lane, and in vector registers (the compiler sees no
+// constants, so that each step is one mixed-precision multiply-add): with hi = fp16(h p + t),
+// u = b hi + (a p + k): w1 = fp16(u), truncated, and w2 = fp16(n w1 + u) are mid and lo in columns 8-15, where
+// u = (p 2^15 - hi) 2^11 is exact, and hi and 0 in columns 0-7.
+// An infinite V makes columns 0-7 infinite whatever its key's weight, as neither MFMA multiplies it by 0
+// there: hi is rounded from p 2^15 + 1.25 2^-25, so that it is never 0, and w2's 0 is replaced by 2^-24.
+// mid takes both differences back (k the second; exact but for that 2^-24, 2^-39 of the largest weight,
+// where p >= 2^-15). (Half of hi in either MFMA does that too, but rounds the accumulators twice: 4096
+// keys 4.2e-7 against 2.6e-7.)
+struct DecWeights {
+    float h, t, a, k, b, n;
+    uint32_t w2;
+};
+__device__ __forceinline__ DecWeights dec_weights(int l16) {
+    const bool low = (l16 & 8) != 0;
+    DecWeights w = {kWScale, 1.25f * 0x1p-25f, low ? kWScale * kLoScale : 0.f, low ? -0x1p-24f * kLoScale : 0.f,
+                    low ? -kLoScale : 1.f, -1.f, low ? 0u : 0x00010001u};
+    asm("" : "+v"(w.h), "+v"(w.t), "+v"(w.a), "+v"(w.k), "+v"(w.b), "+v"(w.n), "+v"(w.w2));
+    return w;
+}
+
+// One 32-key block: scores, online softmax (base 2), PV product. scale2: |sm_scale| log2(e), not 0 (of a
+// negative scale q carries the sign). tok0 / tok1: (wave-uniform) token index of the two pages' first
+// slots; keys outside [tb, te) are masked (a padding page: tok1 >= te). A masked key weighs 0 and, since
+// 0 * NaN is not 0, its V elements are zeroed as well: slots the cache never filled may hold any bits. Its
+// K row only feeds its own score, which is replaced.
+// The running maximum is an unscaled score, and a key's exponent is (score - m) scale2: never above 0,
+// and as accurate for large scores as for small ones (with the scaled scores rounded first, q eight
+// times N(0, 1): error of the output against 64 bits 6.7e-7 at 8192 keys, G = 8).
 __device__ __forceinline__ void dec_block(DecState& st, DecBlock& b, const pf16x8 (&q)[4], int tok0, int tok1,
-                                          int tb, int te, float scale2, float lo_a, float lo_b, int lg) {
+                                          int tb, int te, float scale2, const DecWeights& wc, int lg) {
     float x[8];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -235,7 +270,7 @@ __device__ __forceinline__ void dec_block(DecState& st, DecBlock& b, const pf16x
             c[i] = mfma16x16x32(b.k[t][2 * i + 1], q[2 * i + 1],
                                 mfma16x16x32(b.k[t][2 * i], q[2 * i], pf32x4{0.f, 0.f, 0.f, 0.f}));
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x[4 * t + j] = (c[0][j] + c[1][j]) * scale2;
+        for (int j = 0; j < 4; ++j) x[4 * t + j] = c[0][j] + c[1][j];
     }
     if (tok0 < tb || tok0 + kPage > te || tok1 + kPage > te) {   // wave-uniform: an edge block
         uint32_t keep[4] = {0u, 0u, 0u, 0u};
@@ -258,25 +293,40 @@ __device__ __forceinline__ void dec_block(DecState& st, DecBlock& b, const pf16x
     for (int e = 1; e < 8; ++e) mx = fmaxf(mx, x[e]);
     const float mn = fmaxf(st.m, col4_reduce<true>(mx));
     if (__builtin_amdgcn_ballot_w64(mn > st.m)) {
-        const float al = mn > st.m ? __builtin_amdgcn_exp2f(st.m - mn) : 1.f;
+        const float al = mn > st.m ? __builtin_amdgcn_exp2f((st.m - mn) * scale2) : 1.f;
         st.l *= al;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) st.acc[dt] *= al;
         st.m = mn;
     }
     const float ms = st.m == -INFINITY ? 0.f : st.m;
-    pf16x8 pb;
+    pf16x8 w1, w2;
     float sum = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float p = __builtin_amdgcn_exp2f(x[e] - ms);
-        sum += p;
-        const _Float16 hi = (_Float16)p;
-        pb[e] = (_Float16)fmaf((float)hi, lo_b, p * lo_a);
+    for (int e = 0; e < 8; e += 2) {
+        float u[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float p = __builtin_amdgcn_exp2f((x[e + i] - ms) * scale2);
+            sum += p;
+            u[i] = fmaf((float)(_Float16)fmaf(p, wc.h, wc.t), wc.b, fmaf(p, wc.a, wc.k));
+        }
+        const auto w = __builtin_amdgcn_cvt_pkrtz(u[0], u[1]);   // (truncating: w2 takes what is left either way)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            w1[e + i] = (_Float16)w[i];
+            w2[e + i] = (_Float16)fmaf((float)w[i], wc.n, u[i]);
+        }
     }
     st.l += sum;
+    pu32x4 w2b = __builtin_bit_cast(pu32x4, w2);
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) st.acc[dt] = mfma16x16x32(b.v[dt], pb, st.acc[dt]);
+    for (int i = 0; i < 4; ++i) w2b[i] |= wc.w2;
+    w2 = __builtin_bit_cast(pf16x8, w2b);
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) st.acc[dt] = mfma16x16x32(b.v[dt], w1, st.acc[dt]);
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) st.acc[dt] = mfma16x16x32(b.v[dt], w2, st.acc[dt]);
 }
 
 // End of a segment: the waves of a kv head hand their states (maximum, sum, output) to LDS, and
@@ -286,16 +336,16 @@ __device__ __forceinline__ void dec_block(DecState& st, DecBlock& b, const pf16x
 // barrier suffices: a buffer is written again two flushes later, after the barrier of the next.
 template <class C, int LAY, class ArgP>
 __device__ __forceinline__ void dec_flush(DecShared<C, LAY>& S, DecState& st, int par, ArgP a,
-                                          size_t row0, int slot) {
+                                          size_t row0, int slot, float scale2) {
     typedef DecShared<C, LAY> Sh;
     constexpr int G = C::G, HG = Sh::HG, WPH = C::WPH;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int l16 = lane & 15, lg = lane >> 4, w0 = wave / WPH * WPH;
     const int ltid = tid - w0 * 64;
     const float L = col4_reduce<false>(st.l);
-    // High plus scaled low halves (in columns 0-7).
+    // The parts together, still times 2^15 (in columns 0-7).
     float o[8][4], top = 0.f, ks = 1.f / kLoScale;
-    asm("" : "+v"(ks));   // (in a register: the exchange then folds into the multiply-add)
+    asm("" : "+v"(ks));
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
@@ -304,8 +354,8 @@ __device__ __forceinline__ void dec_flush(DecShared<C, LAY>& S, DecState& st, in
             o[dt][j] = fmaf(dec_ror8(hi), ks, hi);
             top = fmaxf(top, fabsf(hi));
         }
-    // An infinite V makes the high half infinite and the low half NaN (0 * inf, inf - inf): the high
-    // half is then the answer.
+    // An infinite V makes columns 0-7 infinite and columns 8-15 NaN or infinite of either sign (mid and lo
+    // may be 0 or negative): the first are then the answer.
     if (__builtin_amdgcn_ballot_w64(top == INFINITY)) {
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt)
@@ -340,7 +390,7 @@ __device__ __forceinline__ void dec_flush(DecShared<C, LAY>& S, DecState& st, in
             float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int w = 0; w < WPH; ++w) {
-                const float al = mw[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw[w] - M);
+                const float al = mw[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((mw[w] - M) * scale2);
                 const float4 ov = *reinterpret_cast<const float4*>(&S.o[bf][w0 + w][hh][d0]);
                 Ls = fmaf(al, S.l[bf][w0 + w][h], Ls);
                 O.x = fmaf(al, ov.x, O.x);
@@ -348,8 +398,8 @@ __device__ __forceinline__ void dec_flush(DecShared<C, LAY>& S, DecState& st, in
                 O.z = fmaf(al, ov.z, O.z);
                 O.w = fmaf(al, ov.w, O.w);
             }
-            const float ri = Ls > 0.f ? 1.f / Ls : 0.f;
-            const float lse = Ls > 0.f ? (M + __builtin_amdgcn_logf(Ls)) * kDecLn2 : -INFINITY;
+            const float ri = Ls > 0.f ? (1.f / kWScale) / Ls : 0.f;
+            const float lse = Ls > 0.f ? fmaf(M, scale2, __builtin_amdgcn_logf(Ls)) * kDecLn2 : -INFINITY;
             O.x *= ri;
             O.y *= ri;
             O.z *= ri;
