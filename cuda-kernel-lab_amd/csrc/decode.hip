@@ -733,9 +733,15 @@ __device__ __forceinline__ void run_segments(const BalArgs& a, DecShared<C, LAY>
     int sl = 0, nfl = 0;   // the slot of the next block, computed and loaded; loads of the newest block
     const uint8_t* const kc = a.k;
     const uint8_t* const vc = a.v;
-    auto issue = [&]() {
+    // Issues the next block's loads, with step n of `other` (n < 8: the scores of the block just read)
+    // between them: a load takes the issue of 16 cycles, and so does an MFMA.
+    auto issue = [&](auto other) {
         nfl = 0;
-        if (have <= 0) return;
+        if (have <= 0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) other(i);
+            return;
+        }
         nfl = 8 * have + 1;
         const uint32_t lds = lds0 + (uint32_t)(sl * Sh::SLOT);
         if constexpr (NS > 1)
@@ -743,9 +749,12 @@ __device__ __forceinline__ void run_segments(const BalArgs& a, DecShared<C, LAY>
         {
             const size_t off = (size_t)(uint32_t)pid0 * page_bytes + (size_t)pkvh * 256;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) dec_dma(kc + off, koff[i], lds + 1024 * i);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dec_dma(vc + off, voff[i], lds + 2 * kDecPageBytes + 1024 * i);
+            for (int i = 0; i < 8; ++i) {
+                if (i < 4) dec_dma(kc + off, koff[i], lds + 1024 * i);
+                else dec_dma(vc + off, voff[i - 4], lds + 2 * kDecPageBytes + 1024 * (i - 4));
+                other(i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
         if (have > 1) {
             const size_t off = (size_t)(uint32_t)pid1 * page_bytes + (size_t)pkvh * 256;
@@ -755,14 +764,15 @@ __device__ __forceinline__ void run_segments(const BalArgs& a, DecShared<C, LAY>
             for (int i = 0; i < 4; ++i) dec_dma(vc + off, voff[i], lds + 3 * kDecPageBytes + 1024 * i);
         }
     };
+    auto nothing = [](int) {};
 
     PD_STAMP(2);
     advance();
-    issue();
+    issue(nothing);
     advance();
     if constexpr (NS > 1) {
         sl = 1;
-        issue();
+        issue(nothing);
         advance();
         sl = 0;
     }
@@ -796,14 +806,13 @@ __device__ __forceinline__ void run_segments(const BalArgs& a, DecShared<C, LAY>
             }
             dec_read_block(b, S.slot[wave][sl], l16, lg);
             dec_wait_lds();
-            issue();
+            if (NS > 1) dec_sign_q(q, scale);
+            pf32x4 c[2][2];
+            issue([&](int n) { dec_score(c, b, q, n); });
             advance();
-            if (NS > 1) {
-                dec_sign_q(q, scale);
-                sl ^= 1;
-            }
+            if (NS > 1) sl ^= 1;
             const int tok0 = tbase + (lw + WPH * blk) * kPage;
-            dec_block(st, b, q, tok0, blk + 1 < cnt ? tok0 + WPH * kPage : t1, t0, t1, scale2, wc, lg);
+            dec_block(st, b, c, tok0, blk + 1 < cnt ? tok0 + WPH * kPage : t1, t0, t1, scale2, wc, lg, blk == 0);
             if (si == 0 && blk == 0) PD_STAMP(3);
         }
         if (si < 12) PD_STAMP(4 + 2 * si);

@@ -21,8 +21,9 @@
 // Staging: a wave moves its own pages with 16-byte direct global->LDS loads into its own 16 KB slots
 // (K and V of two pages), so the loop has no workgroup barrier. Per block the wave waits for its
 // slot, reads all operands of the block into registers (K rows with ds_read_b128, V with the
-// transposing ds_read_b64_tr_b16), issues the next loads into the slot, and computes. One slot keeps
-// 16 KB per wave, 64 KB per CU, in flight, which covers the loaded latency of long streams; two slots
+// transposing ds_read_b64_tr_b16), issues the next loads into the slot, the score MFMAs between them, and
+// computes. One slot keeps 16 KB per wave, 64 KB per CU, in flight, which covers the loaded latency of
+// long streams; two slots
 // (G <= 4) start short sequences sooner: one sequence of 4096 tokens 9.43 -> 8.93 us, 128 of 16-512
 // at G = 1 96.2 -> 94.6 us, 32768 tokens 27.6 -> 26.8 us; 64 x 1024 41.9 -> 42.1 us.
 //
@@ -250,49 +251,68 @@ __device__ __forceinline__ DecWeights dec_weights(int l16) {
     return w;
 }
 
-// One 32-key block: scores, online softmax (base 2), PV product. scale2: |sm_scale| log2(e), not 0 (of a
-// negative scale q carries the sign). tok0 / tok1: (wave-uniform) token index of the two pages' first
+// The scores of a block, eight MFMAs: step n < 8 of them. Two chains of two per 16 keys: fewer roundings in
+// a row than one of four, and half its latency.
+__device__ __forceinline__ void dec_score(pf32x4 (&c)[2][2], const DecBlock& b, const pf16x8 (&q)[4], int n) {
+    const int k = n >> 2, t = (n >> 1) & 1, i = n & 1;
+    c[t][i] = mfma16x16x32(b.k[t][2 * i + k], q[2 * i + k], k ? c[t][i] : pf32x4{0.f, 0.f, 0.f, 0.f});
+}
+
+// A 32-key block from its scores c: online softmax (base 2), PV product. scale2: |sm_scale| log2(e), not 0
+// (of a negative scale q carries the sign). tok0 / tok1: (wave-uniform) token index of the two pages' first
 // slots; keys outside [tb, te) are masked (a padding page: tok1 >= te). A masked key weighs 0 and, since
 // 0 * NaN is not 0, its V elements are zeroed as well: slots the cache never filled may hold any bits. Its
 // K row only feeds its own score, which is replaced.
 // The running maximum is an unscaled score, and a key's exponent is (score - m) scale2: never above 0,
 // and as accurate for large scores as for small ones (with the scaled scores rounded first, q eight
 // times N(0, 1): error of the output against 64 bits 6.7e-7 at 8192 keys, G = 8).
-__device__ __forceinline__ void dec_block(DecState& st, DecBlock& b, const pf16x8 (&q)[4], int tok0, int tok1,
-                                          int tb, int te, float scale2, const DecWeights& wc, int lg) {
+// A short segment is a block or two per wave, so what only edge blocks and first blocks do counts: a
+// segment's first block (first) has nothing to rescale, and an absent second page is masked without
+// looking at its keys. With the scores between the next loads and the flush's own loads in one trip, GPU
+// time: one sequence of 2048 tokens 7.27 -> 6.98 us, 8 of 94-988 11.9 -> 11.35, 16 of 64-512 at G = 1 and 32
+// kv heads 19.6 -> 19.2.
+__device__ __forceinline__ void dec_block(DecState& st, DecBlock& b, const pf32x4 (&c)[2][2], int tok0, int tok1,
+                                          int tb, int te, float scale2, const DecWeights& wc, int lg, bool first) {
     float x[8];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        // (two chains of two: fewer roundings in a row than one of four, and half its latency)
-        pf32x4 c[2];
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-            c[i] = mfma16x16x32(b.k[t][2 * i + 1], q[2 * i + 1],
-                                mfma16x16x32(b.k[t][2 * i], q[2 * i], pf32x4{0.f, 0.f, 0.f, 0.f}));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) x[4 * t + j] = c[0][j] + c[1][j];
-    }
+        for (int j = 0; j < 4; ++j) x[4 * t + j] = c[t][0][j] + c[t][1][j];
     if (tok0 < tb || tok0 + kPage > te || tok1 + kPage > te) {   // wave-uniform: an edge block
-        uint32_t keep[4] = {0u, 0u, 0u, 0u};
+        if (tok0 >= tb && tok0 + kPage <= te && tok1 >= te) {   // a whole page and none
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int tok = (e < 4 ? tok0 : tok1) + 4 * lg + (e & 3);
-            if (tok >= tb && tok < te) keep[e / 2] |= e & 1 ? 0xFFFF0000u : 0x0000FFFFu;
-            else x[e] = -INFINITY;
-        }
+            for (int e = 4; e < 8; ++e) x[e] = -INFINITY;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-            pu32x4 w = __builtin_bit_cast(pu32x4, b.v[dt]);
+            for (int dt = 0; dt < 8; ++dt) {
+                pu32x4 w = __builtin_bit_cast(pu32x4, b.v[dt]);
+                w[2] = w[3] = 0u;
+                b.v[dt] = __builtin_bit_cast(pf16x8, w);
+            }
+        } else {
+            uint32_t keep[4] = {0u, 0u, 0u, 0u};
+            const uint32_t n = (uint32_t)(te - tb);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) w[i] &= keep[i];
-            b.v[dt] = __builtin_bit_cast(pf16x8, w);
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t k = (uint32_t)((e < 4 ? tok0 : tok1) - tb + 4 * lg + (e & 3));
+                if (k < n) keep[e / 2] |= e & 1 ? 0xFFFF0000u : 0x0000FFFFu;
+                else x[e] = -INFINITY;
+            }
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) {
+                pu32x4 w = __builtin_bit_cast(pu32x4, b.v[dt]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] &= keep[i];
+                b.v[dt] = __builtin_bit_cast(pf16x8, w);
+            }
         }
     }
     float mx = x[0];
 #pragma unroll
     for (int e = 1; e < 8; ++e) mx = fmaxf(mx, x[e]);
     const float mn = fmaxf(st.m, col4_reduce<true>(mx));
-    if (__builtin_amdgcn_ballot_w64(mn > st.m)) {
+    if (first) {   // (wave-uniform)
+        st.m = mn;
+    } else if (__builtin_amdgcn_ballot_w64(mn > st.m)) {
         const float al = mn > st.m ? __builtin_amdgcn_exp2f((st.m - mn) * scale2) : 1.f;
         st.l *= al;
 #pragma unroll
@@ -342,6 +362,10 @@ __device__ __forceinline__ void dec_flush(DecShared<C, LAY>& S, DecState& st, in
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int l16 = lane & 15, lg = lane >> 4, w0 = wave / WPH * WPH;
     const int ltid = tid - w0 * 64;
+    // where the rows go (read from the kernel arguments here, in the time of the arithmetic before the barrier)
+    void* const dst = slot < 0 ? (void*)a->out : (void*)a->part_o;
+    float* const dst_lse = slot < 0 ? a->lse : a->part_lse;
+    const int ps = a->part_stride;
     const float L = col4_reduce<false>(st.l);
     // The parts together, still times 2^15 (in columns 0-7).
     float o[8][4], top = 0.f, ks = 1.f / kLoScale;
@@ -378,25 +402,30 @@ __device__ __forceinline__ void dec_flush(DecShared<C, LAY>& S, DecState& st, in
         }
         dec_barrier();
 #pragma unroll
-        for (int idx = ltid; idx < HG * 32; idx += WPH * 64) {
-            const int hh = idx / 32, h = hp * HG + hh, d0 = 4 * (idx % 32);
-            float mw[WPH], M = -INFINITY;
+        for (int i = 0; i < (HG * 32 + WPH * 64 - 1) / (WPH * 64); ++i) {
+            const int idx = ltid + i * WPH * 64;
+            if ((i + 1) * WPH * 64 > HG * 32 && idx >= HG * 32) break;
+            const int hh = idx >> 5, h = hp * HG + hh, d0 = 4 * (idx & 31);
+            float mw[WPH], lw[WPH], M = -INFINITY;
+            float4 ov[WPH];
 #pragma unroll
             for (int w = 0; w < WPH; ++w) {
                 mw[w] = S.m[bf][w0 + w][h];
-                M = fmaxf(M, mw[w]);
+                lw[w] = S.l[bf][w0 + w][h];
+                ov[w] = *reinterpret_cast<const float4*>(&S.o[bf][w0 + w][hh][d0]);
             }
+#pragma unroll
+            for (int w = 0; w < WPH; ++w) M = fmaxf(M, mw[w]);
             float Ls = 0.f;
             float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int w = 0; w < WPH; ++w) {
                 const float al = mw[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((mw[w] - M) * scale2);
-                const float4 ov = *reinterpret_cast<const float4*>(&S.o[bf][w0 + w][hh][d0]);
-                Ls = fmaf(al, S.l[bf][w0 + w][h], Ls);
-                O.x = fmaf(al, ov.x, O.x);
-                O.y = fmaf(al, ov.y, O.y);
-                O.z = fmaf(al, ov.z, O.z);
-                O.w = fmaf(al, ov.w, O.w);
+                Ls = fmaf(al, lw[w], Ls);
+                O.x = fmaf(al, ov[w].x, O.x);
+                O.y = fmaf(al, ov[w].y, O.y);
+                O.z = fmaf(al, ov[w].z, O.z);
+                O.w = fmaf(al, ov[w].w, O.w);
             }
             const float ri = Ls > 0.f ? (1.f / kWScale) / Ls : 0.f;
             const float lse = Ls > 0.f ? fmaf(M, scale2, __builtin_amdgcn_logf(Ls)) * kDecLn2 : -INFINITY;
@@ -404,16 +433,14 @@ __device__ __forceinline__ void dec_flush(DecShared<C, LAY>& S, DecState& st, in
             O.y *= ri;
             O.z *= ri;
             O.w *= ri;
+            const size_t e = slot < 0 ? row0 + h : ps > 0 ? (row0 + h) * (size_t)ps + slot : (size_t)slot * G + h;
             if (slot < 0) {
                 const pf16x4 hv = {(_Float16)O.x, (_Float16)O.y, (_Float16)O.z, (_Float16)O.w};
-                *reinterpret_cast<pf16x4*>(a->out + (row0 + h) * kHeadDim + d0) = hv;
-                if (d0 == 0) a->lse[row0 + h] = lse;
+                *reinterpret_cast<pf16x4*>(static_cast<_Float16*>(dst) + e * kHeadDim + d0) = hv;
             } else {
-                const int ps = a->part_stride;
-                const size_t e = ps > 0 ? (row0 + h) * (size_t)ps + slot : (size_t)slot * G + h;
-                *reinterpret_cast<float4*>(a->part_o + e * kHeadDim + d0) = O;
-                if (d0 == 0) a->part_lse[e] = lse;
+                *reinterpret_cast<float4*>(static_cast<float*>(dst) + e * kHeadDim + d0) = O;
             }
+            if (d0 == 0) dst_lse[e] = lse;
         }
         if (Sh::NB == 1 || hp + 1 < G / HG) dec_barrier();
     }
