@@ -364,11 +364,20 @@ class Plan:
 
     def run(self, q, k_cache, v_cache, kv_indptr, kv_indices, kv_last_page_len, out, lse,
             workspace, nbytes: int, sm_scale=None, stream=None):
-        # (a decode step calls this once per layer: the native function is looked up once, and the scale
-        # is converted by the call itself)
-        st = self._run(self._h, ptr(q), ptr(k_cache), ptr(v_cache), ptr(kv_indptr), ptr(kv_indices),
-                       ptr(kv_last_page_len), _SCALE if sm_scale is None else sm_scale, ptr(out), ptr(lse),
-                       ptr(workspace), nbytes, stream_ptr(stream))
+        # A decode step calls this once per layer, and a small one is bound by the host: the native function
+        # is looked up once, the scale converted by the call itself, and tensors (and a torch stream) taken
+        # without the type tests of ptr() and stream_ptr(), which are for everything else. Nothing has been
+        # called when either exception comes.
+        sc = _SCALE if sm_scale is None else sm_scale
+        try:
+            st = self._run(self._h, q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), kv_indptr.data_ptr(),
+                           kv_indices.data_ptr(), kv_last_page_len.data_ptr(), sc, out.data_ptr(),
+                           lse.data_ptr(), workspace.data_ptr(), nbytes,
+                           None if stream is None else stream.cuda_stream)
+        except (AttributeError, ctypes.ArgumentError):
+            st = self._run(self._h, ptr(q), ptr(k_cache), ptr(v_cache), ptr(kv_indptr), ptr(kv_indices),
+                           ptr(kv_last_page_len), sc, ptr(out), ptr(lse), ptr(workspace), nbytes,
+                           stream_ptr(stream))
         if st:
             _check(st, "pdattn_plan_run")
 

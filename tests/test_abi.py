@@ -197,3 +197,34 @@ def test_cascade_prefix_rejects_chunk_sizes(chunk_tokens):
     with pytest.raises(pdattn.PdattnError) as e:
         pdattn.cascade_prefix(pp)
     assert e.value.status == 2   # PDATTN_ERR_UNSUPPORTED
+
+
+def test_plan_run_takes_every_kind_of_pointer():
+    """Plan.run takes tensors without type tests and everything else (ints, None, objects whose data_ptr()
+    is another integer type, a stream as an int, an object or None) as ptr() does. The plan was never
+    uploaded, so the native call refuses before it looks at any of them."""
+    import numpy as np
+    import torch
+
+    class Address:
+        def __init__(self, v):
+            self.v = v
+
+        def data_ptr(self):
+            return np.int64(self.v)
+
+    class Stream:
+        cuda_stream = np.int64(0)
+
+    plan = pdattn.Plan([0, 2], [16], 1, 8, 8, force_workgroups=8)
+    t = torch.zeros(64, dtype=torch.float16)
+    for kind in (t, 4096, None, Address(4096)):
+        for scale in (None, 0.5, np.float32(0.5), 1):
+            for stream in (None, 0, Stream()):
+                with pytest.raises(pdattn.PdattnError) as e:
+                    plan.run(t, kind, t, t, kind, t, t, t, kind, 1 << 20, scale, stream)
+                assert e.value.status == {v: k for k, v in pdattn.STATUS.items()}["PDATTN_ERR_NOT_READY"]
+    for bad in ("text", 1.5, object()):
+        with pytest.raises((AttributeError, ctypes.ArgumentError, TypeError)):
+            plan.run(t, bad, t, t, t, t, t, t, t, 1 << 20)
+    plan.close()
