@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <cstdlib>
 
+#include "launch_rules.h"
 #include "pdattn_internal.h"
 #include "timeline.h"
 
@@ -1412,7 +1413,7 @@ hipError_t launch_decode_ranges(const DevArgs& a, int G, int hp, hipStream_t s) 
 
 hipError_t launch_merge_ranges(const DevMergeArgs& a, hipStream_t s) {
     if (a.B <= 0) return hipSuccess;
-    return launch_merge(a.ngroups / a.B + 2, (int64_t)a.B * a.Hq, [&](auto u, auto wide, dim3 grid, dim3 block) {
+    return launch_merge(merge_ranges_sources(a.ngroups, a.B), (int64_t)a.B * a.Hq, [&](auto u, auto wide, dim3 grid, dim3 block) {
         merge_ranges_kernel<decltype(u)::value, decltype(wide)::value><<<grid, block, 0, s>>>(a);
     });
 }
