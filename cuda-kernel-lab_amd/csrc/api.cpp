@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "../../include/pdattn.h"
+#include "launch_rules.h"
 #include "pdattn_internal.h"
 
 using namespace pdattn;
@@ -971,14 +972,10 @@ static int launch_uniform_split(const PartialArgs& a, int G, hipStream_t s) {
     }
     DeviceFacts f;
     if (int st = device_facts(&f)) return st;
-    // An item is one chunk of hp kv heads: two where that still fills the CUs (8 x 8192 tokens in 4
-    // chunks, 256 items of one head or 128 of two: 47.9 against 54.1 us).
-    const int hp = a.Hkv % 2 == 0 && (int64_t)a.num_chunks * a.B * a.Hkv >= 2 * f.cus ? 2 : 1;
-    const int64_t n_items = (int64_t)a.num_chunks * a.B * (a.Hkv / hp);
-    if (n_items > (int64_t)1 << 30) return fail(PDATTN_ERR_INVALID_ARGUMENT, "too many chunks");
-    const int64_t slots = (int64_t)f.cus;
-    int64_t per = (n_items + slots - 1) / slots;
-    per = std::max<int64_t>(1, std::min<int64_t>({per, (int64_t)kSegMax, kRangeMax / ppi}));
+    const int64_t chunks = (int64_t)a.num_chunks * a.B;
+    if (chunks > (int64_t)1 << 30) return fail(PDATTN_ERR_INVALID_ARGUMENT, "too many chunks");
+    const UniformSplit us = uniform_split(chunks, a.Hkv, f.cus, std::min<int64_t>(kSegMax, kRangeMax / ppi));
+    if (us.items > (int64_t)1 << 30) return fail(PDATTN_ERR_INVALID_ARGUMENT, "too many chunks");
     UniArgs u;
     BalArgs& d = u.d;
     d.q = a.q;
@@ -993,7 +990,7 @@ static int launch_uniform_split(const PartialArgs& a, int G, hipStream_t s) {
     d.B = a.B;
     d.Hq = a.Hq;
     d.Hkv = a.Hkv;
-    d.W = (int)((n_items + per - 1) / per);
+    d.W = (int)us.W;
     d.scale_log2 = a.scale_log2;
     d.part_stride = a.part_stride;
     d.ngroups = 0;
@@ -1005,9 +1002,9 @@ static int launch_uniform_split(const PartialArgs& a, int G, hipStream_t s) {
     u.chunk_tokens = a.chunk_tokens;
     u.num_chunks = a.num_chunks;
     u.chunk_base = a.chunk_base;
-    u.n_items = (int)n_items;
-    u.per_wg = (int)per;
-    PD_HIP(launch_decode_uniform(u, G, hp, s));
+    u.n_items = (int)us.items;
+    u.per_wg = (int)us.per;
+    PD_HIP(launch_decode_uniform(u, G, us.hp, s));
     return PDATTN_OK;
 }
 

@@ -13,4 +13,30 @@ namespace pdattn {
 // 200-6000 73.2 / 72.4 / 72.9 / 73.7.
 inline int merge_ranges_sources(int ngroups, int B) { return std::min(ngroups, std::max(ngroups / B + 2, 16)); }
 
+// The uniform split's launch: `chunks` (chunk, sequence) pairs of Hkv kv heads as items of hp heads of one
+// chunk, `per` items per workgroup, W workgroups. A workgroup holds at most seg_max items.
+struct UniformSplit {
+    int hp;
+    int64_t items, per, W;
+};
+inline UniformSplit uniform_items(int64_t chunks, int Hkv, int hp, int64_t cus, int64_t seg_max) {
+    const int64_t items = chunks * (Hkv / hp);
+    const int64_t per = std::max<int64_t>(1, std::min((items + cus - 1) / cus, seg_max));
+    return {hp, items, per, (items + per - 1) / per};
+}
+// One or two heads per item: two read 512 contiguous bytes of every token row, which streams faster, but
+// make the items twice as long, so that the last round of workgroups may leave more of the chip idle. Two
+// need items enough for every CU (8 x 8192 tokens in 4 chunks: 47.9 us with one head, 54.1 with two); then
+// they are taken unless the longest workgroup grows by more than a quarter and fewer than three quarters of
+// the CUs have one. Chunks of 1024 tokens, 8 kv heads, one / two heads: 65 sequences 49.3 / 54.4 us, 88
+// 58.4 / 61.3, 96 65.8 / 65.1, 100 74.2 / 67.2; 200 of 300 tokens 45.4 / 43.6, 140 of 256 30.4 / 28.0; 17 of
+// 1024 with 32 kv heads 51.1 / 53.3.
+inline UniformSplit uniform_split(int64_t chunks, int Hkv, int64_t cus, int64_t seg_max) {
+    const UniformSplit one = uniform_items(chunks, Hkv, 1, cus, seg_max);
+    if (Hkv % 2 != 0 || one.items < 2 * cus) return one;
+    const UniformSplit two = uniform_items(chunks, Hkv, 2, cus, seg_max);
+    auto longest = [&](const UniformSplit& u) { return (u.W + cus - 1) / cus * u.per * u.hp; };
+    return 4 * longest(two) <= 5 * longest(one) || 4 * two.W >= 3 * cus ? two : one;
+}
+
 }  // namespace pdattn

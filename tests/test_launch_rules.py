@@ -25,3 +25,34 @@ def test_merge_trips_fit_the_longest_row(rules):
             assert 1 <= n <= ngroups
             assert -(-ngroups // n) <= 4, (ngroups, B, n)
             assert n >= min(ngroups, ngroups // B + 2)
+
+
+def _uniform(rules, chunks, Hkv, cus=256, seg_max=24):
+    out = (ctypes.c_int64 * 4)()
+    rules.rule_uniform_split(ctypes.c_int64(chunks), Hkv, ctypes.c_int64(cus), ctypes.c_int64(seg_max), out)
+    return list(out)
+
+
+def test_uniform_split_covers_the_items(rules):
+    for Hkv in (1, 2, 3, 8, 16, 32):
+        for chunks in list(range(1, 300)) + [1000, 4097, 100000]:
+            for seg_max in (1, 7, 24):
+                hp, items, per, W = _uniform(rules, chunks, Hkv, seg_max=seg_max)
+                assert hp in (1, 2) and Hkv % hp == 0 and items * hp == chunks * Hkv
+                assert 1 <= per <= seg_max and (W - 1) * per < items <= W * per
+
+
+def test_two_heads_per_item_leave_no_more_of_the_chip_idle(rules):
+    """Two heads where the longest workgroup is at most a quarter longer or three quarters of the CUs
+    have one; never with fewer items than would keep every CU busy."""
+    for Hkv in (2, 8, 32):
+        for chunks in range(1, 1200):
+            hp, items, per, W = _uniform(rules, chunks, Hkv)
+            if hp == 1:
+                continue
+            assert items >= 256
+            one = min(24, -(-chunks * Hkv // 256))
+            assert W >= 192 or 2 * per <= 1.25 * one or W > 256, (Hkv, chunks)
+    assert [_uniform(rules, n, 8)[0] for n in (32, 65, 88, 96, 100, 140, 200)] == [1, 1, 1, 2, 2, 2, 2]
+    assert _uniform(rules, 17, 32)[0] == 1
+    assert _uniform(rules, 64, 7)[0] == 1
