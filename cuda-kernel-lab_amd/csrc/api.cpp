@@ -1123,13 +1123,13 @@ int dev_layout(const pdattn_decode_params* p, int G, DevLayout* L) {
     }
     DeviceFacts f;
     if (int st = device_facts(&f)) return st;
-    // one workgroup per CU of one kv head, or of two (as the plan path), whole groups of Hkv; more ranges if a
-    // range could hold more pages than the kernel stages (kRangeMax): every sequence attends at
-    // most ceil(span / 16) + 1 pages
+    // one workgroup per CU of one kv head, or of two, whole groups of Hkv; more ranges if a range could
+    // hold more pages than the kernel stages (kRangeMax): every sequence attends at most
+    // ceil(span / 16) + 1 pages
     L->span = (int64_t)p->num_chunks * p->chunk_tokens;
     const int64_t per_seq = L->span / kPage + 2;
     const int64_t bound = (int64_t)p->B * per_seq;
-    L->hp = p->Hkv % 2 == 0 ? 2 : 1;
+    L->hp = device_range_heads(p->B, per_seq, p->Hkv, f.cus);
     int64_t NG = std::max<int64_t>(1, (int64_t)f.cus * L->hp / p->Hkv);
     NG = std::max<int64_t>(NG, (bound + kRangeMax - 1) / kRangeMax);
     if (NG * p->Hkv > (1 << 24)) return fail(PDATTN_ERR_INVALID_ARGUMENT, "too many ranges");

@@ -39,4 +39,16 @@ inline UniformSplit uniform_split(int64_t chunks, int Hkv, int64_t cus, int64_t 
     return 4 * longest(two) <= 5 * longest(one) || 4 * two.W >= 3 * cus ? two : one;
 }
 
+// Kv heads per workgroup of the device-range decode over `cus` CUs. Two heads stream faster but double the
+// ranges, and so the partials of every long sequence; the lengths are not known here, only that a sequence
+// attends at most per_seq pages. Two from 16 such pages per range on (about 8 real ones in a ragged batch,
+// as in a plan), or with more sequences than ranges of one head; never for one sequence. One / two heads,
+// us: 1 x 2048 tokens 9.0 / 9.7, 1 x 32768 28.3 / 28.8, 4 of 200-900 11.2 / 11.6, 8 of 94-988 12.4 / 12.6,
+// with 32 kv heads 19.2 / 18.7, 32 of 200-6000 73.2 / 72.4, one of 30000 and 15 of 200 33.5 / 32.4.
+inline int device_range_heads(int64_t B, int64_t per_seq, int Hkv, int64_t cus) {
+    if (Hkv % 2 != 0 || B < 2) return 1;
+    const int64_t ranges = std::max<int64_t>(1, cus / Hkv);
+    return B * per_seq >= 16 * 2 * ranges || B > ranges ? 2 : 1;
+}
+
 }  // namespace pdattn

@@ -56,3 +56,15 @@ def test_two_heads_per_item_leave_no_more_of_the_chip_idle(rules):
     assert [_uniform(rules, n, 8)[0] for n in (32, 65, 88, 96, 100, 140, 200)] == [1, 1, 1, 2, 2, 2, 2]
     assert _uniform(rules, 17, 32)[0] == 1
     assert _uniform(rules, 64, 7)[0] == 1
+
+
+def test_device_ranges_of_short_batches_keep_one_head(rules):
+    """Two heads only where every range holds enough pages, or there are more sequences than ranges."""
+    def heads(B, longest, Hkv, cus=256):
+        return rules.rule_device_range_heads(ctypes.c_int64(B), ctypes.c_int64(longest // 16 + 2), Hkv,
+                                             ctypes.c_int64(cus))
+    assert [heads(1, n, 8) for n in (16, 2048, 32768, 200000)] == [1, 1, 1, 1]
+    assert [heads(B, 988, 8) for B in (2, 4, 8, 17, 32)] == [1, 1, 1, 2, 2]
+    assert heads(32, 6000, 8) == 2 and heads(33, 16, 8) == 2 and heads(32, 16, 8) == 1
+    assert heads(8, 988, 32) == 2 and heads(64, 4096, 7) == 1
+    assert heads(300, 16, 512) == 2   # more kv heads than CUs
