@@ -1239,7 +1239,7 @@ int pdattn_plan_get_info(const pdattn_plan* pl, pdattn_plan_info* info) {
     info->chunk_pages = pl->P;
     info->segments = pl->segments;
     info->merge_entries = pl->n_entries;
-    info->paired = pl->hp > 1 && pl->G <= 4 && pl->n_entries == 0 ? 1 : 0;
+    info->paired = pl->hp > 1 ? 1 : 0;
     info->schedule_ints = (int)schedule_ints(pl);
     return PDATTN_OK;
 }

@@ -194,16 +194,16 @@ typedef struct pdattn_plan_info {
     int     segments;          /* segments over all workgroups                            */
     int     merge_entries;     /* pairs merged by the second launch (0: single launch)    */
     int     schedule_ints;     /* int32 count of pdattn_plan_get_schedule's output        */
-    int     paired;            /* 1: a G <= 4 plan of two workgroups per CU (w and w + 1, kv heads
-                                  2k, 2k + 1 of one page range, run as one kernel workgroup)
-                                  that splits no sequence over workgroups; 0 for every other
-                                  plan, also where kernel workgroups hold two heads          */
+    int     paired;            /* 1: the decode launch runs workgroups w and w + 1 (kv heads
+                                  2k, 2k + 1 of one page range) as one, workgroups / 2 in all;
+                                  0: one launched workgroup for each                        */
 } pdattn_plan_info;
 
 /* Build a plan from host copies of kv_indptr [B+1] and kv_last_page_len [B]. force_workgroups > 0
  * overrides the grid size (by default one workgroup per CU, or two where Hkv is even and the batch
- * has 8 pages per range or more sequences than ranges: the kernel then runs workgroups w and w + 1, kv heads 2k and 2k + 1 of one
- * page range, as one; it grows when a workgroup would exceed its segment or page limits).
+ * has 8 pages per range or more sequences than ranges: the kernel then runs workgroups w and w + 1,
+ * kv heads 2k and 2k + 1 of one page range, as one (info.paired); it grows when a workgroup would
+ * exceed its segment or page limits).
  * chunk_pages > 0, or a grid that is not a
  * multiple of Hkv, selects the other partition: chunks of up to chunk_pages pages (64 by default)
  * of one (sequence, kv head) pair, ordered sequence-major, then by chunk position, kv head

@@ -1,12 +1,12 @@
-"""GPU parity of the paired decode kernel against the fp64 oracle, through the C ABI.
+"""GPU parity of plans that run two kv heads per workgroup against the fp64 oracle, through the C ABI.
 
-A default page-range plan at G <= 4 with an even Hkv is first built with two plan workgroups per
-CU; when it splits no sequence, the decode launch runs plan workgroups w and w + 1 (kv heads 2k and
-2k + 1 of the same page range) as one 4-wave workgroup whose pages go through LDS (info.paired).
-Cases: the metric's 64x1K shape at G = 4, 2 and 1; many sequences per range (several segments per
-workgroup); partial last pages with NaN / Inf in every slot past a sequence's end; Hkv = 2;
-bitwise determinism; a workspace the caller wrote over (the kernel leaves out / lse alone); and
-the shapes that must not be paired (a split sequence, G = 8, an odd Hkv).
+A default page-range plan of an even Hkv has two plan workgroups per CU where the batch holds 8 pages per
+range or more sequences than ranges; the decode launch then runs plan workgroups w and w + 1 (kv heads
+2k and 2k + 1 of the same page range) as one 4-wave workgroup (info.paired). Cases: the metric's 64x1K
+shape at G = 4, 2 and 1; many sequences per range (several segments per workgroup); partial last pages
+with NaN / Inf in every slot past a sequence's end; Hkv = 2; sequences split over workgroups and G = 8;
+bitwise determinism; a workspace the caller wrote over (the kernel leaves out / lse alone); and the
+batches that are not paired (an odd Hkv, few pages and sequences, a forced grid).
 """
 import numpy as np
 import pytest
@@ -151,20 +151,44 @@ def test_paired_workspace_written_by_the_caller(what):
     B.close()
 
 
-NOT_PAIRED = [
-    ("1x32K (the paired plan would split it)", [32768], 32, 8, 14),
+PAIRED_SPLIT = [
+    ("1x32K", [32768], 32, 8, 14),
     ("G=8", [1024] * 64, 64, 8, 15),
-    ("odd Hkv", [1024] * 64, 12, 3, 16),
+    ("G=8, split", [700, 30000, 33, 0, 5000], 64, 8, 17),
+    ("9 sequences of a few pages, 32 heads", [40, 5, 333, 16, 1, 100, 77, 400, 250], 32, 32, 18),
 ]
 
 
-@pytest.mark.parametrize("name,lens,Hq,Hkv,seed", NOT_PAIRED, ids=[c[0] for c in NOT_PAIRED])
-def test_not_paired(name, lens, Hq, Hkv, seed):
+@pytest.mark.parametrize("name,lens,Hq,Hkv,seed", PAIRED_SPLIT, ids=[c[0] for c in PAIRED_SPLIT])
+def test_paired_plans_that_split_sequences_or_hold_eight_heads(name, lens, Hq, Hkv, seed):
     import _gpu
-    print(f"[case] unpaired plan: {name}", flush=True)
+    _need_256_cus()
+    print(f"[case] paired plan: {name}", flush=True)
     bt = inputs.make_batch(lens, Hq, Hkv, seed=seed)
     ro, rl = _ref(bt)
     o, l, info = _gpu.run_plan(_gpu.DeviceBatch(bt))
+    assert info.paired == 1 and info.workgroups % 2 == 0
+    assert info.merge_entries > 0 or "split" not in name
+    check_out(o, ro, tag=name)
+    check_lse(l, rl, tag=name)
+
+
+NOT_PAIRED = [
+    ("odd Hkv", [1024] * 64, 12, 3, 16, 0),
+    ("few pages", [2048], 32, 8, 19, 0),
+    ("few pages, several sequences", [500, 17, 900], 64, 8, 20, 0),
+    ("a forced grid", [1024] * 64, 32, 8, 21, 512),
+]
+
+
+@pytest.mark.parametrize("name,lens,Hq,Hkv,seed,wg", NOT_PAIRED, ids=[c[0] for c in NOT_PAIRED])
+def test_not_paired(name, lens, Hq, Hkv, seed, wg):
+    import _gpu
+    _need_256_cus()
+    print(f"[case] unpaired plan: {name}", flush=True)
+    bt = inputs.make_batch(lens, Hq, Hkv, seed=seed)
+    ro, rl = _ref(bt)
+    o, l, info = _gpu.run_plan(_gpu.DeviceBatch(bt), wg)
     assert info.paired == 0
     check_out(o, ro, tag=name)
     check_lse(l, rl, tag=name)

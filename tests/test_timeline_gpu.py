@@ -1,7 +1,7 @@
 """The timeline build of the library (make -C cuda-kernel-lab_amd timeline: the kernels compiled
 with per-workgroup timestamps, read by bench.py --timeline) computes exactly what the library
-proper computes, and its stamps come in phase order: the plan path's decode (one kv head per
-workgroup, and the paired kernel), the fused cascade step (decode and prefix roles, then the
+proper computes, and its stamps come in phase order: the plan path's decode (one kv head per workgroup, and
+two, with as many launched workgroups as the plan's info says), the fused cascade step (decode and prefix roles, then the
 merge) and the prefix kernel alone with a partial last chunk (its 4-wave and key-split bodies),
 each compared bit for bit.
 
@@ -46,31 +46,31 @@ CHILD = textwrap.dedent(r"""
     L.pdattn_timeline_read_decode.argtypes = [ctypes.c_void_p, ctypes.c_size_t]
     buf = np.zeros(8192 * 32, np.uint64)
     assert L.pdattn_timeline_read_decode(buf.ctypes.data, buf.nbytes) == 0
-    t = buf.reshape(8192, 32)[:info.workgroups].astype(np.int64)
+    t = buf.reshape(8192, 32).astype(np.int64)
     ran = t[:, 0] > 0
-    assert ran.sum() > 0
+    assert ran.sum() == info.workgroups // (1 + info.paired), "info does not count the launched workgroups"
     for row in t[ran]:
         seq = [row[0], row[1], row[2]] + [row[s] for s in range(4, 28) if row[s] > 0] + [row[31]]
         assert all(b >= a for a, b in zip(seq, seq[1:])), f"stamps out of order: {seq}"
     print("ok", int(ran.sum()), "workgroups stamped", flush=True)
 
-    # the paired kernel (a plan that splits no sequence: 64 x 1024 tokens on 256 CUs)
-    print("[case] paired kernel, timeline build vs library, 64 x 1024", flush=True)
-    bq = inputs.make_batch([1024] * 64, 32, 8, seed=52)
-    _, o0, l0, i0 = run(lib0, bq)
-    pdattn._lib = None
-    pdattn.LIB_PATH = sys.argv[2]
-    assert pdattn.lib().pdattn_timeline_reset_decode() == 0   # (no stamps left from the case above)
-    L, o1, l1, i1 = run(sys.argv[2], bq)
-    assert np.array_equal(o0, o1) and np.array_equal(l0, l1), "timeline build changed the paired results"
-    assert i0.paired == i1.paired
-    if i1.paired:
+    # two kv heads per workgroup: whole sequences, G = 8, a split sequence (256 CUs)
+    for lens, Hq in (([1024] * 64, 32), ([1024] * 64, 64), ([32768], 32)):
+        print(f"[case] paired plan, timeline build vs library, {len(lens)} x {lens[0]} Hq={Hq}", flush=True)
+        bq = inputs.make_batch(lens, Hq, 8, seed=52)
+        _, o0, l0, i0 = run(lib0, bq)
+        pdattn._lib = None
+        pdattn.LIB_PATH = sys.argv[2]
+        assert pdattn.lib().pdattn_timeline_reset_decode() == 0   # (no stamps left from the case above)
+        L, o1, l1, i1 = run(sys.argv[2], bq)
+        assert np.array_equal(o0, o1) and np.array_equal(l0, l1), "timeline build changed the paired results"
+        assert i0.paired == i1.paired
         # (a new handle: its functions need their argument types again, or the pointer is cut to an int)
         L.pdattn_timeline_read_decode.argtypes = [ctypes.c_void_p, ctypes.c_size_t]
         assert L.pdattn_timeline_read_decode(buf.ctypes.data, buf.nbytes) == 0
-        t = buf.reshape(8192, 32)[:i1.workgroups // 2].astype(np.int64)
+        t = buf.reshape(8192, 32).astype(np.int64)
         ran = t[:, 0] > 0
-        assert ran.sum() > 0
+        assert ran.sum() == i1.workgroups // (1 + i1.paired), "info does not count the launched workgroups"
         for row in t[ran]:
             seq = [row[0], row[1], row[2]] + [row[s] for s in range(4, 28) if row[s] > 0] + [row[31]]
             assert all(b >= a for a, b in zip(seq, seq[1:])), f"paired stamps out of order: {seq}"
