@@ -1369,7 +1369,7 @@ int pdattn_cascade_plan_get_info(const pdattn_cascade_plan* cp, pdattn_cascade_i
     info->prefix_tokens = cp->Lp;
     info->prefix_chunks = cp->n_extra;
     info->prefix_workgroups = cp->n_items * cp->base.Hkv;
-    info->suffix_workgroups = cp->sk.W;
+    info->suffix_workgroups = cp->sk.W / cp->sk.hp;   // launched
     info->workspace_bytes = cp->ws_bytes;
     info->nodes = (int)cp->nodes.size();
     info->levels = cp->levels;

@@ -300,8 +300,8 @@ typedef struct pdattn_cascade_info {
     int    use;             /* 1 when a shared prefix of >= min_prefix tokens was found  */
     int    prefix_tokens;   /* Lp (of the first node)                                   */
     int    prefix_chunks;   /* prefix partial slots per row                            */
-    int    prefix_workgroups;
-    int    suffix_workgroups;
+    int    prefix_workgroups;  /* launched for the prefix pass                            */
+    int    suffix_workgroups;  /* and for the suffix decode (of one or two kv heads each)  */
     size_t workspace_bytes;
     int    nodes;           /* shared-prefix nodes (1 for the reference's rule)        */
     int    levels;          /* depth of the node tree                                  */

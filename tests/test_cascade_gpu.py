@@ -338,25 +338,27 @@ def test_fused_mode_at_g8_and_unknown_mode():
     check_lse(l, rl)
 
 
-@pytest.mark.parametrize("n,Hq,Hkv", [(3500, 8, 2), (1200, 32, 4)], ids=["G4", "G8"])
-def test_many_short_sequences_grow_the_suffix_grid(n, Hq, Hkv):
-    """n sequences of 1..16 private tokens behind a 64-token prefix: the (sequence, kv head) pairs
-    need more than one suffix workgroup per CU (at most 24 segments each, 8 at G=8, where the
-    fused step's decode role stages q rows for 8), so the fused step's prefix blocks start after a
-    grid larger than the CU count."""
+@pytest.mark.parametrize("n,Hq,Hkv,launched", [(3500, 8, 2, 256), (6500, 8, 2, 512), (3300, 32, 4, 512)],
+                         ids=["G4", "G4 grown", "G8 grown"])
+def test_many_short_sequences_grow_the_suffix_grid(n, Hq, Hkv, launched):
+    """n sequences of 1..16 private tokens behind a 64-token prefix, two kv heads per workgroup: a
+    workgroup holds at most 24 segments, so more than 24 sequences per default range (512 / Hkv ranges)
+    need more than one suffix workgroup per CU, and the fused step's prefix blocks start after a grid
+    larger than the CU count; fewer do not."""
+    import torch
     import _gpu
     import pdattn
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("cases sized for 256 CUs")
     rng = np.random.default_rng(64)
     suffix = [int(x) for x in rng.integers(1, 17, size=n)]
     bt = inputs.make_shared_prefix_batch(64, suffix, Hq, Hkv, seed=64)
     db = _gpu.DeviceBatch(bt)
     print(f"cascade: {n} short sequences G={bt.G}", flush=True)
-    cp = pdattn.CascadePlan(db.params(), bt.indptr, bt.indices, bt.lens, db.indices, 16)
-    info = cp.info()
-    cp.close()
-    assert info.use == 1 and info.mode == pdattn.CASCADE_FUSED
-    assert info.suffix_workgroups > pdattn.device_info().compute_units
+    assert (n > 24 * 512 // Hkv) == (launched > 256)
     o, l, info = _gpu.run_cascade(db, min_prefix=16)
+    assert info.use == 1 and info.mode == pdattn.CASCADE_FUSED
+    assert info.suffix_workgroups == launched
     ro, rl = _ref(bt)
     check_out(o, ro)
     check_lse(l, rl)
