@@ -93,10 +93,13 @@ UNIFORM_SHAPES = [
     # tag, lens, Hq, Hkv, num_chunks, chunk_tokens, kv_start
     ("chunk past the LDS page list", [40000, 123], 32, 8, 1, 40000, 0),   # 2501 pages: one-chunk kernel
     ("long chunks", [40000, 123], 32, 8, 2, 20000, 0),
-    ("many items per workgroup", "ragged300", 8, 8, 1, 304, 0),         # 2400 items, 10 per workgroup
-    ("segment cap per workgroup", "ragged300", 8, 8, 3, 100, 0),        # 7200 items, 24 per workgroup
+    ("many items per workgroup", "ragged300", 8, 8, 1, 304, 0),         # 1200 two-head items, 5 per workgroup
+    ("15 items per workgroup", "ragged300", 8, 8, 3, 100, 0),           # 3600 two-head items
+    ("segment cap per workgroup", "ragged300", 8, 8, 6, 50, 0),         # 7200 two-head items, 24 per workgroup
+    ("segment cap, one head per item", "ragged300", 28, 7, 4, 75, 0),   # 8400 one-head items, 24 per workgroup
     ("unaligned start and chunk", [1000, 77, 0, 513], 32, 8, 5, 200, 23),
-    ("G=8, segment cap of the compact layout", "ragged300", 64, 8, 2, 160, 0),   # 4800 items, 8 per workgroup
+    ("G=8, 10 items per workgroup", "ragged300", 64, 8, 2, 160, 0),     # 2400 two-head items
+    ("G=8, segment cap per workgroup", "ragged300", 64, 8, 6, 50, 0),   # 7200 two-head items, 24 per workgroup
 ]
 
 

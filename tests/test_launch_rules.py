@@ -68,3 +68,9 @@ def test_device_ranges_of_short_batches_keep_one_head(rules):
     assert heads(32, 6000, 8) == 2 and heads(33, 16, 8) == 2 and heads(32, 16, 8) == 1
     assert heads(8, 988, 32) == 2 and heads(64, 4096, 7) == 1
     assert heads(300, 16, 512) == 2   # more kv heads than CUs
+
+
+def test_items_per_workgroup_of_the_parity_cases(rules):
+    """What the uniform split's GPU parity cases say they cover (300 sequences, 256 CUs)."""
+    assert [_uniform(rules, 300 * nc, 8)[:3:2] for nc in (1, 2, 3, 6)] == [[2, 5], [2, 10], [2, 15], [2, 24]]
+    assert _uniform(rules, 300 * 4, 7)[:3:2] == [1, 24]
