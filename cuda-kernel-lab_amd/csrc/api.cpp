@@ -256,7 +256,7 @@ struct pdattn_plan {
     int split_pairs = 0, max_contrib = 0, n_entries = 0, n_slots = 0, segments = 0;
     int cmax = 0;                     // > 0: partial slots laid out by merge entry (e * cmax + k)
     int hp = 1;                       // kv heads per kernel workgroup (W / hp workgroups)
-    uint32_t range_q = 0, range_r = 0, range_m = 0, hkv_m = 0;   // ranges without divisions (BalArgs)
+    RangeConsts rc;                   // of a page-range plan
     // workspace layout (bytes from the base)
     size_t off_desc = 0, off_list = 0, off_plse = 0, off_po = 0, ws_bytes = 0;
     int stride = 8;                   // ints per descriptor block
@@ -420,10 +420,7 @@ int build_balanced_plan(const int32_t* indptr, const int32_t* last, int B, int H
         pl->P = (int)((nnz + W / Hkv - 1) / (W / Hkv));   // pages per range
         pl->ngroups = (int)(W / Hkv);
         pl->hp = hp;   // (W = NG Hkv is even: plan workgroups 2 x and 2 x + 1 share range g)
-        pl->range_q = (uint32_t)(nnz / pl->ngroups);
-        pl->range_r = (uint32_t)(nnz % pl->ngroups);
-        pl->range_m = 0xFFFFFFFFu / (uint32_t)pl->ngroups;
-        pl->hkv_m = 0xFFFFFFFFu / (uint32_t)Hkv;
+        pl->rc = range_consts(nnz, pl->ngroups, Hkv);
     }
     for (; !grouped;) {
         wsegs.assign((size_t)W, 0);
@@ -597,10 +594,7 @@ BalArgs bal_args(const pdattn_plan* pl, const void* q, const void* k, const void
     a.tag = pl->tag;
     a.desc_stride = pl->stride;
     a.qrow_b = pl->ngroups > 0 && pl->B == 1 ? 0 : -1;
-    a.range_q = pl->range_q;
-    a.range_r = pl->range_r;
-    a.range_m = pl->range_m;
-    a.hkv_m = pl->hkv_m;
+    a.rc = pl->rc;
     return a;
 }
 

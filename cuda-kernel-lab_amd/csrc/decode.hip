@@ -853,9 +853,9 @@ __device__ __forceinline__ void balanced_body(const BalArgs& a, DecShared<C, LAY
         // descriptor block(s), in round trip 1.
         uint32_t g = 0, lo = 0, npr = 0;
         if constexpr (RANGES) {
-            g = dec_div((uint32_t)w, (uint32_t)a.Hkv, a.hkv_m);
-            lo = dec_range(a, g);
-            npr = min(dec_range(a, g + 1) - lo, (uint32_t)DecShared<C, LAY>::PGMAX);
+            g = div_by((uint32_t)w, (uint32_t)a.Hkv, a.rc.hkv_m);
+            lo = range_start(a.rc, a.nnz, a.ngroups, g);
+            npr = min(range_start(a.rc, a.nnz, a.ngroups, g + 1) - lo, (uint32_t)DecShared<C, LAY>::PGMAX);
             qpre = DecShared<C, LAY>::NS == 1 && a.qrow_b >= 0;
         }
         const int dst = a.desc_stride;   // <= kBalDescInts <= NT

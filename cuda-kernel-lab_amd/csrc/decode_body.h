@@ -77,18 +77,6 @@ struct DecShared {
     int sd[C::HP][kBalDescInts];         // descriptor block(s): header, then segments
 };
 
-// x / d for x < 2^32 without a division, m = floor((2^32 - 1) / d): the high product is the quotient or
-// one less.
-__device__ __forceinline__ uint32_t dec_div(uint32_t x, uint32_t d, uint32_t m) {
-    const uint32_t t = (uint32_t)(((uint64_t)x * m) >> 32);
-    return t + ((t + 1) * (uint64_t)d <= x ? 1u : 0u);
-}
-// nnz g / ngroups (g <= ngroups) of a page-range plan
-__device__ __forceinline__ uint32_t dec_range(const BalArgs& a, uint32_t g) {
-    if (a.ngroups < 65536) return a.range_q * g + dec_div(a.range_r * g, (uint32_t)a.ngroups, a.range_m);
-    return (uint32_t)((uint64_t)a.nnz * g / (uint32_t)a.ngroups);
-}
-
 // The segment fields of a descriptor block (8 ints each) through a window of 8 segments in one
 // register: field f of segment si is a lane read, and LDS is read once per 8 segments.
 struct SegWin {

@@ -8,6 +8,8 @@
 
 #include "../../include/pdattn.h"
 
+#include "range_arith.h"
+
 namespace pdattn {
 
 constexpr int kHeadDim = 128;
@@ -72,9 +74,7 @@ struct BalArgs {
     // qrow_b, so a workgroup's q rows (kv head w % Hkv) are loaded with its descriptor block
     int qrow_b = -1;
     int desc_stride = 0;          // ints per descriptor block (header and the most segments of a block)
-    // ranges and kv heads of a page-range plan without a division: nnz / ngroups, nnz % ngroups, and
-    // floor((2^32 - 1) / d) for d = ngroups and d = Hkv
-    uint32_t range_q = 0, range_r = 0, range_m = 0, hkv_m = 0;
+    RangeConsts rc;               // ranges and kv heads of a page-range plan without a division
 };
 
 // The reference-shaped uniform split (decode_partial / decode_attention) run by the balanced

@@ -23,3 +23,14 @@ def oracle_lib():
     import oracle
     oracle.build()
     return oracle
+
+
+@pytest.fixture(scope="session")
+def host_rules(tmp_path_factory):
+    """The dispatch rules and range arithmetic of csrc/, compiled with the host compiler."""
+    import ctypes
+    import subprocess
+    so = str(tmp_path_factory.mktemp("rules") / "launch_rules.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC",
+                    os.path.join(ROOT, "tests", "cpp", "launch_rules.cpp"), "-o", so], check=True)
+    return ctypes.CDLL(so)

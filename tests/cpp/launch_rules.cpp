@@ -1,5 +1,7 @@
-// The dispatch rules of csrc/launch_rules.h behind C functions, for tests/test_launch_rules.py.
+// The dispatch rules of csrc/launch_rules.h and the range arithmetic of csrc/range_arith.h behind C
+// functions, for tests/test_launch_rules.py and tests/test_range_arithmetic.py.
 #include "../../cuda-kernel-lab_amd/csrc/launch_rules.h"
+#include "../../cuda-kernel-lab_amd/csrc/range_arith.h"
 
 extern "C" {
 
@@ -16,6 +18,15 @@ void rule_uniform_split(int64_t chunks, int Hkv, int64_t cus, int64_t seg_max, i
 
 int rule_device_range_heads(int64_t B, int64_t per_seq, int Hkv, int64_t cus) {
     return pdattn::device_range_heads(B, per_seq, Hkv, cus);
+}
+
+uint32_t rule_div(uint32_t x, uint32_t d) { return pdattn::div_by(x, d, pdattn::div_multiplier(d)); }
+uint32_t rule_range_start(int64_t nnz, int ngroups, int Hkv, uint32_t g) {
+    return pdattn::range_start(pdattn::range_consts(nnz, ngroups, Hkv), nnz, ngroups, g);
+}
+// w / Hkv as the kernel works it out
+uint32_t rule_group_of(uint32_t w, int64_t nnz, int ngroups, int Hkv) {
+    return pdattn::div_by(w, (uint32_t)Hkv, pdattn::range_consts(nnz, ngroups, Hkv).hkv_m);
 }
 
 }

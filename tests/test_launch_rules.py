@@ -1,19 +1,12 @@
 """The host's dispatch rules (csrc/launch_rules.h, compiled here with the host compiler) -- CPU only."""
 import ctypes
-import os
-import subprocess
 
 import pytest
 
-HERE = os.path.dirname(os.path.abspath(__file__))
 
-
-@pytest.fixture(scope="module")
-def rules(tmp_path_factory):
-    so = str(tmp_path_factory.mktemp("rules") / "launch_rules.so")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC",
-                    os.path.join(HERE, "cpp", "launch_rules.cpp"), "-o", so], check=True)
-    return ctypes.CDLL(so)
+@pytest.fixture
+def rules(host_rules):
+    return host_rules
 
 
 def test_merge_trips_fit_the_longest_row(rules):
