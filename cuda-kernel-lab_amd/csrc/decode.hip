@@ -474,11 +474,9 @@ __device__ __forceinline__ void merge_load(const MSrc& A, const MSrc& B, int k0,
     for (int u = 0; u < U; ++u) {
         const int k = min(k0 + r + 8 * u, n - 1);
         const bool inA = k < A.n;
-        const size_t i = inA ? (size_t)k * A.stride : (size_t)(k - A.n) * B.stride;
-        const float* lp = inA ? A.lse : B.lse;
-        const float* op = inA ? A.o : B.o;
-        l[u] = lp[i];
-        o[u] = *reinterpret_cast<const float4*>(op + i * kHeadDim + d0);
+        const size_t ia = (size_t)k * A.stride, ib = (size_t)(k - A.n) * B.stride;
+        l[u] = *(inA ? A.lse + ia : B.lse + ib);
+        o[u] = *reinterpret_cast<const float4*>((inA ? A.o + ia * kHeadDim : B.o + ib * kHeadDim) + d0);
     }
 }
 // Folds this lane's loaded sources into s in order, branch-free (a dropped or empty source weighs 0
@@ -1189,28 +1187,24 @@ __global__ __launch_bounds__(kMergeThreads) void merge_ranges_kernel(DevMergeArg
     const int row = merge_row<WIDE>(), d0 = merge_d0<WIDE>(), b = row / a.Hq, hq = row - b * a.Hq;
     const int kvh = hq / a.G, hh = hq - kvh * a.G;
     const int64_t pb = a.prefix[b], pe = a.prefix[b + 1], N = a.prefix[a.B];
-    MState st{-INFINITY, 0.f, make_float4(0.f, 0.f, 0.f, 0.f)};
+    MSrc A{a.part_lse, a.part_o, 1, 0}, Bs = A;   // (no source: the fold leaves the empty state, out 0, lse -inf)
     if (pe > pb) {
         const int64_t NG = a.ngroups;
         const int64_t g0 = ((pb + 1) * NG - 1) / N, g1 = (pe * NG - 1) / N;
         if (g0 == g1) return;
         const size_t i0 = ((size_t)(g0 * a.Hkv + kvh) * 2 + 1) * a.G + hh;       // slot 2 w + 1 of g0
         const size_t i1 = ((size_t)((g0 + 1) * a.Hkv + kvh) * 2) * a.G + hh;     // slot 2 w of g0 + 1
-        const MSrc A{a.part_lse + i0, a.part_o + i0 * kHeadDim, 1, 1};
-        const MSrc Bs{a.part_lse + i1, a.part_o + i1 * kHeadDim, (size_t)2 * a.Hkv * a.G, (int)(g1 - g0)};
-        st = merge_lanes<U>(A, Bs, d0, [](int) { return true; });
-    } else {
-        // (the fold leaves the empty state: out 0, lse -inf)
-        const MSrc E{a.part_lse, a.part_o, 1, 0};
-        st = merge_lanes<U>(E, E, d0, [](int) { return true; });
+        A = MSrc{a.part_lse + i0, a.part_o + i0 * kHeadDim, 1, 1};
+        Bs = MSrc{a.part_lse + i1, a.part_o + i1 * kHeadDim, (size_t)2 * a.Hkv * a.G, (int)(g1 - g0)};
     }
+    const MState st = merge_lanes<U>(A, Bs, d0, [](int) { return true; });
     merge_store(st, d0, a.out + (size_t)row * kHeadDim, a.lse + row);
 }
 
 // One kv head per workgroup (C::HP = 1), or HP neighbouring heads of a page-range plan: workgroup x
 // runs the plan's workgroups HP x .. HP x + HP - 1.
 template <class C, bool RANGES>
-__global__ __launch_bounds__(C::NT, 2) void decode_balanced_kernel(BalArgs a) {
+__global__ __launch_bounds__(C::NT, 1) void decode_balanced_kernel(BalArgs a) {
     __shared__ DecShared<C, kLayWide> S;
     balanced_body<C, false, kLayWide, RANGES>(a, S, blockIdx.x);
 }
@@ -1218,14 +1212,14 @@ __global__ __launch_bounds__(C::NT, 2) void decode_balanced_kernel(BalArgs a) {
 // The reference-shaped uniform split on the balanced body (items of equal key ranges, descriptors
 // built in the kernel from the device page table).
 template <class C>
-__global__ __launch_bounds__(C::NT, 2) void decode_uniform_kernel(UniArgs u) {
+__global__ __launch_bounds__(C::NT, 1) void decode_uniform_kernel(UniArgs u) {
     __shared__ DecShared<C, kLayWide> S;
     balanced_body<C, true>(u.d, S, blockIdx.x, &u);
 }
 
 // The drop-in decode_attention over page ranges found on the device.
 template <class C>
-__global__ __launch_bounds__(C::NT, 2) void decode_ranges_kernel(DevArgs d) {
+__global__ __launch_bounds__(C::NT, 1) void decode_ranges_kernel(DevArgs d) {
     __shared__ DevShared<C> S;
     dev_body<C>(d, S, blockIdx.x);
 }
