@@ -16,15 +16,13 @@
 //  * A uniform chunk too long for the runner's LDS page list runs on decode_partial_kernel, one
 //    workgroup per (sequence, kv head, chunk), on the vector unit:
 //    - K and V rows go straight from HBM into VGPRs with 16-byte non-temporal loads: a 256-byte row
-//      (128 fp16) is read by LPR lanes, so one wave-wide load instruction reads 64/LPR rows of one
-//      page, each as whole 128-byte lines; a two-page ring, one page in flight;
+//      (128 fp16) is read by 16 lanes, so one wave-wide load instruction reads 4 rows of one page, each
+//      as whole 128-byte lines; a two-page ring, one page in flight;
 //    - each lane takes the fp16 dot product of its slice of q_h and k_j with v_dot2_f32_f16, and the
-//      LPR lanes of a row sum with DPP row ops, which leaves the score in every lane of the row;
-//    - every lane keeps its own online-softmax state over the keys it holds; the 64/LPR states of a
+//      16 lanes of a row sum with DPP row ops, which leaves the score in every lane of the row;
+//    - every lane keeps its own online-softmax state over the keys it holds; the four states of a
 //      wave are merged once at the end, and the waves of the workgroup through LDS.
-//    LPR = 16 lanes per row, 4 rows per wave-wide load, each lane holding 4 rows x 8 dims of a page.
-//    Lane (r = lane / LPR, c = lane % LPR) holds rows i*RPI + r of each page and the 16-byte pieces
-//    kk*LPR + c (dims 8*(kk*LPR + c) .. +7), kk < PPL.
+//    Lane (r = lane / 16, c = lane % 16) holds rows 4 i + r of each page and dims 8 c .. 8 c + 7.
 //  * Softmax runs in base 2 on log2(e)-prescaled scores with v_exp_f32 / v_log_f32
 //    (exp(x) = 2^(x log2 e)); the running output is rescaled only when some max grows (a
 //    wave-uniform branch), which after the first pages is rare.
@@ -51,10 +49,10 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.69314718055994531f;
 
 // Compile-time shape of a decode kernel instance.
-template <int G_, int LPR_, int NW_, int NBUF_>
+template <int G_, int NW_, int NBUF_>
 struct Cfg {
     static constexpr int G = G_;                   // query heads per kv head
-    static constexpr int LPR = LPR_;               // lanes per 256-byte K/V row (8 or 16)
+    static constexpr int LPR = 16;                 // lanes per 256-byte K/V row
     static constexpr int NW = NW_;                 // waves per workgroup
     static constexpr int NBUF = NBUF_;             // pages held in VGPRs per wave (NBUF-1 in flight)
     static constexpr int NT = NW * 64;
@@ -70,9 +68,9 @@ __device__ __forceinline__ float dpp(float v) {
         float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
 }
 
-// Sums over the LPR lanes that share one K/V row (a DPP row is 16 lanes) of N independent values, one
+// Sums over the 16 lanes (a DPP row) that share one K/V row of N independent values, one
 // DPP step at a time across all of them.
-template <int LPR, int N>
+template <int N>
 __device__ __forceinline__ void row_sum_all(float* v) {
 #pragma unroll
     for (int j = 0; j < N; ++j) v[j] += dpp<0xB1>(v[j]);
@@ -80,15 +78,12 @@ __device__ __forceinline__ void row_sum_all(float* v) {
     for (int j = 0; j < N; ++j) v[j] += dpp<0x4E>(v[j]);
 #pragma unroll
     for (int j = 0; j < N; ++j) v[j] += dpp<0x141>(v[j]);
-    if constexpr (LPR == 16) {
 #pragma unroll
-        for (int j = 0; j < N; ++j) v[j] += dpp<0x140>(v[j]);
-    }
+    for (int j = 0; j < N; ++j) v[j] += dpp<0x140>(v[j]);
 }
 
-// Combine of the 64/LPR row groups of a wave (lanes LPR apart hold the same head dims), leaving
-// the result in every lane: row_ror:8 pairs the two groups of a 16-lane row (LPR = 8), then
-// v_permlane16_swap / v_permlane32_swap pair whole 16-lane rows, all in the VALU. After
+// Combine of the four row groups of a wave (lanes 16 apart hold the same head dims), leaving the result
+// in every lane: v_permlane16_swap / v_permlane32_swap pair whole 16-lane rows, all in the VALU. After
 // swap(a, b) the two results hold, in every lane, the values of both rows of its pair (rows
 // r and r^1 for the 16-lane swap, r and r^2 for the 32-lane swap), always in the same order, so
 // r0 + r1 is bitwise the same in all lanes. The second operand is passed through an empty asm
@@ -121,18 +116,14 @@ __device__ __forceinline__ f16x2 as_h2(uint32_t w) { return __builtin_bit_cast(f
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 
-template <int LPR>
 __device__ __forceinline__ float xgroup_sum(float v) {
     float a, b;
-    if constexpr (LPR == 8) v += dpp<0x128>(v);   // row_ror:8
     row_pair<false>(v, a, b);
     row_pair<true>(a + b, a, b);
     return a + b;
 }
-template <int LPR>
 __device__ __forceinline__ float xgroup_max(float v) {
     float a, b;
-    if constexpr (LPR == 8) v = fmaxf(v, dpp<0x128>(v));
     row_pair<false>(v, a, b);
     row_pair<true>(fmaxf(a, b), a, b);
     return fmaxf(a, b);
@@ -223,7 +214,7 @@ __device__ __forceinline__ void page_step(WaveState<C>& st, PageRegs<C>& pr,
                                                  false);
             x[i][h] = acc;
         }
-    row_sum_all<g::LPR, g::RG * G>(&x[0][0]);
+    row_sum_all<g::RG * G>(&x[0][0]);
 #pragma unroll
     for (int i = 0; i < g::RG; ++i) {
         const int tok = tok_r + i * g::RPI;
@@ -351,14 +342,14 @@ __device__ __forceinline__ void process_range(Smem<C::G, C::NW>& sm, const _Floa
         }
     }
 
-    // merge the 64/LPR row-group states of this wave (lanes LPR apart hold the same dims)
+    // merge the four row-group states of this wave (lanes 16 apart hold the same dims)
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-        const float M = xgroup_max<g::LPR>(st.m[h]);
+        const float M = xgroup_max(st.m[h]);
         const float a = (st.m[h] == -INFINITY) ? 0.f : fast_exp2(st.m[h] - M);
-        st.l[h] = xgroup_sum<g::LPR>(st.l[h] * a);
+        st.l[h] = xgroup_sum(st.l[h] * a);
 #pragma unroll
-        for (int d = 0; d < g::DPL; ++d) st.o[h][d] = xgroup_sum<g::LPR>(st.o[h][d] * a);
+        for (int d = 0; d < g::DPL; ++d) st.o[h][d] = xgroup_sum(st.o[h][d] * a);
         st.m[h] = M;
     }
     if (lane < g::LPR) {
@@ -411,12 +402,12 @@ __device__ __forceinline__ KArgPtr kargs() {
 
 // ---- merging partial states ----------------------------------------------------------------
 // Log-sum-exp merge of one row (128 dims) from partial states in a fixed order (merge_states,
-// 01_decode_attention.cu:238-255), by one workgroup of kMergeThreads = 4 waves, with no LDS and no
-// barrier. The sources are two lists, A then B (a pair's partial slots, then a cascade row's prefix
+// 01_decode_attention.cu:238-255), by one workgroup of kMergeThreads = 4 waves (or four of one wave,
+// merge_d0 below), with no LDS and no barrier. The sources are two lists, A then B (a pair's partial slots, then a cascade row's prefix
 // partials): source k of a list has its lse at lse[k * stride] and its output row at
 // o[k * stride * 128]. Wave w covers dims [32 w, 32 w + 32): lane 8 q + r holds the 4 dims
-// 32 w + 4 q .. of sources r, r + 8, r + 16, ... of each list. The first 32 sources of both lists
-// are loaded before any is waited for (one round trip), each lane folds its sources in order (A's,
+// 32 w + 4 q .. of sources r, r + 8, r + 16, ... of the two lists as one. 8 U sources (U chosen at the
+// launch) are loaded before any is waited for (one round trip), each lane folds its sources in order (A's,
 // then B's), and the 8 source lanes of a quad are then combined by three DPP exchanges (lane
 // distances 1, 2, then the other quad of the 8-lane half row): a fixed order, so the result is
 // deterministic. keepA(k), evaluated after the loads, drops source k of A (a slot the decode launch
@@ -1225,8 +1216,8 @@ __global__ __launch_bounds__(C::NT, 1) void decode_ranges_kernel(DevArgs d) {
 }
 
 // The fused cascade step: blocks [0, n_dec) are the suffix decode's workgroups, the rest the
-// prefix pass's (item x, kv head) workgroups. Both roles are 4-wave workgroups of about 210
-// VGPRs and 69 KB of LDS, so a CU holds one of each: the dispatcher places the first n_dec blocks
+// prefix pass's (item x, kv head) workgroups. Both roles are 4-wave workgroups of at most 256 VGPRs
+// and half the LDS, so a CU holds one of each: the dispatcher places the first n_dec blocks
 // one per CU, and the prefix blocks fill the second slots, so every CU streams suffix pages
 // while its matrix core works on the prefix. Partials of both go to the workspace and are merged
 // by the next launch.
@@ -1235,6 +1226,7 @@ __global__ __launch_bounds__(C::NT, 2) void cascade_step_kernel(StepArgs s) {
     static_assert(C::NT == kPrefixThreads, "both roles use the same workgroup shape");
     typedef DecShared<C, kLayStep> Dec;
     constexpr size_t SB = sizeof(Dec) > sizeof(PSmem) ? sizeof(Dec) : sizeof(PSmem);
+    static_assert(2 * SB <= 160 * 1024, "a CU's LDS holds two of these workgroups");
     __shared__ __align__(256) unsigned char raw[SB];
     const int i = blockIdx.x;
     if (i < s.n_dec) {
@@ -1253,11 +1245,10 @@ int occupancy_of(const void* fn, int threads) {
 
 // Kernel shapes per group size G.
 // One-chunk-per-workgroup kernel (the uniform split's fallback for chunks past the LDS page list):
-// 16 lanes per 256-byte row, 4 waves, a two-page ring. Against 8 lanes per row and 8 waves (the
-// planner then picks half the chunks, by occupancy), measured cold when it ran every uniform
-// split: 64x1K 57.0 vs 64.3 us, 1x32K 39.9 vs 39.8 us, 8x8K 57.2 vs 57.8 us.
+// 16 lanes per 256-byte row, 4 waves, a two-page ring. Against 8 lanes per row and 8 waves, measured
+// cold when it ran every uniform split: 64x1K 57.0 vs 64.3 us, 1x32K 39.9 vs 39.8 us, 8x8K 57.2 vs 57.8 us.
 template <int G>
-using PartialCfg = Cfg<G, 16, 4, 2>;
+using PartialCfg = Cfg<G, 4, 2>;
 // MFMA body (plan/run, the uniform split, device ranges and the cascade's suffix): one kv head per
 // 4-wave workgroup, or two neighbouring heads of a page range, two waves each.
 template <int G>
@@ -1327,7 +1318,10 @@ hipError_t launch_decode_partial(const PartialArgs& a, int G, hipStream_t s) {
 }
 
 // The merge kernels: `n` sources per row (the most, or about as many) choose how many a lane loads in
-// one round trip, so that short lists load nothing twice and long ones take one trip.
+// one round trip, so that short lists load nothing twice and long ones take one trip, and up to 64 rows
+// (one or two sequences) run on four times as many CUs. Against 32 per trip in 4-wave workgroups always: 1
+// x 32768 tokens (32 rows of 64 sources) 26.8 -> 25.9 us, 64 ragged sequences at G = 8 (2944 rows of 2
+// or 3 sources) 93.8 -> 92.0.
 template <class F>
 hipError_t launch_merge(int n, int64_t rows, F launch) {
     const bool wide = rows <= 64;
