@@ -1434,24 +1434,25 @@ int pdattn_cascade_decode(pdattn_cascade_plan* cp, void* out, float* lse, pdattn
     a.col0 = 0;
     a.scale_log2 = p.sm_scale * 1.4426950408889634f;
     char* skb = base + cp->off_sk;
-    if (cp->mode == PDATTN_CASCADE_FUSED) {
-        // one launch: the suffix decode's workgroups, then the prefix workgroups beside them
-        if (!res_holds(skb + cp->sk.off_desc, schedule_bytes(&cp->sk), cp->sk.id))
-            return fail(PDATTN_ERR_NOT_READY, "suffix plan was not uploaded into this workspace");
-        StepArgs sa;
-        sa.d = bal_args(&cp->sk, p.q, p.k_cache, p.v_cache, sidx, p.sm_scale, out, lse, skb);
-        sa.p = a;
-        sa.n_dec = cp->sk.U > 0 ? cp->sk.W / cp->sk.hp : 0;
-        sa.n_pre = cp->n_items * p.Hkv;
-        PD_HIP(launch_cascade_step(sa, p.Hq / p.Hkv, cp->sk.hp, s));
+    if (cp->mode == PDATTN_CASCADE_SERIAL) {
+        PD_HIP(launch_cascade_prefix(a, p.Hq / p.Hkv, s));
         return run_plan(&cp->sk, p.q, p.k_cache, p.v_cache, sind, sidx, p.kv_last_page_len, p.sm_scale,
-                        out, lse, skb, cp->sk.ws_bytes, s, ppo, pplse, cp->n_extra, nullptr, false);
+                        out, lse, skb, cp->sk.ws_bytes, s, ppo, pplse, cp->n_extra);
     }
-    // Separate launches. Two streams: the prefix launch runs on the plan's second stream while
-    // the suffix decode runs on `s`; `s` waits for it before the merge, so the step stays one
-    // fork / join (graph-capturable).
+    // Fused: one launch, the suffix decode's workgroups, then the prefix workgroups beside them. Two
+    // streams: the prefix launch runs on the plan's second stream while the suffix decode runs on `s`;
+    // `s` waits for it before the merge, so the step stays one fork / join (graph-capturable). The
+    // suffix then is the fused step without its prefix workgroups, whose smaller LDS leaves a CU room
+    // for one of those (with the plan path's decode kernel, which takes a CU's LDS, the passes ran one
+    // after the other: 64 x (8192 + 512) tokens 70.0 us, 32 x 16384 at G = 8 80.1).
     const bool two = cp->mode == PDATTN_CASCADE_TWO_STREAMS;
-    hipStream_t ps = s;
+    if (!res_holds(skb + cp->sk.off_desc, schedule_bytes(&cp->sk), cp->sk.id))
+        return fail(PDATTN_ERR_NOT_READY, "suffix plan was not uploaded into this workspace");
+    StepArgs sa;
+    sa.d = bal_args(&cp->sk, p.q, p.k_cache, p.v_cache, sidx, p.sm_scale, out, lse, skb);
+    sa.p = a;
+    sa.n_dec = cp->sk.U > 0 ? cp->sk.W / cp->sk.hp : 0;
+    sa.n_pre = two ? 0 : cp->n_items * p.Hkv;
     if (two) {
         if (!cp->aux) {
             PD_HIP(hipStreamCreateWithFlags(&cp->aux, hipStreamNonBlocking));
@@ -1460,13 +1461,12 @@ int pdattn_cascade_decode(pdattn_cascade_plan* cp, void* out, float* lse, pdattn
         }
         PD_HIP(hipEventRecord(cp->ev_fork, s));
         PD_HIP(hipStreamWaitEvent(cp->aux, cp->ev_fork, 0));
-        ps = cp->aux;
+        PD_HIP(launch_cascade_prefix(a, p.Hq / p.Hkv, cp->aux));
+        PD_HIP(hipEventRecord(cp->ev_join, cp->aux));
     }
-    PD_HIP(launch_cascade_prefix(a, p.Hq / p.Hkv, ps));
-    if (two) PD_HIP(hipEventRecord(cp->ev_join, ps));
+    PD_HIP(launch_cascade_step(sa, p.Hq / p.Hkv, cp->sk.hp, s));
     return run_plan(&cp->sk, p.q, p.k_cache, p.v_cache, sind, sidx, p.kv_last_page_len, p.sm_scale,
-                    out, lse, skb, cp->sk.ws_bytes, s, ppo, pplse, cp->n_extra,
-                    two ? cp->ev_join : nullptr);
+                    out, lse, skb, cp->sk.ws_bytes, s, ppo, pplse, cp->n_extra, two ? cp->ev_join : nullptr, false);
 }
 
 int pdattn_cascade_set_mode(pdattn_cascade_plan* cp, int mode) {
