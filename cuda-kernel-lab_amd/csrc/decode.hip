@@ -1202,10 +1202,10 @@ __global__ __launch_bounds__(C::NT, 1) void decode_balanced_kernel(BalArgs a) {
 
 // The reference-shaped uniform split on the balanced body (items of equal key ranges, descriptors
 // built in the kernel from the device page table).
-template <class C>
+template <class C, int LAY>
 __global__ __launch_bounds__(C::NT, 1) void decode_uniform_kernel(UniArgs u) {
-    __shared__ DecShared<C, kLayWide> S;
-    balanced_body<C, true>(u.d, S, blockIdx.x, &u);
+    __shared__ DecShared<C, LAY> S;
+    balanced_body<C, true, LAY>(u.d, S, blockIdx.x, &u);
 }
 
 // The drop-in decode_attention over page ranges found on the device.
@@ -1270,8 +1270,13 @@ void launch_pair(const BalArgs& a, hipStream_t s) {
     decode_balanced_kernel<C, true><<<a.W / C::HP, C::NT, 0, s>>>(a);
 }
 template <class C>
-void launch_u(const UniArgs& a, hipStream_t s) {
-    decode_uniform_kernel<C><<<a.d.W, C::NT, 0, s>>>(a);
+void launch_u(const UniArgs& a, bool two_slots, hipStream_t s) {
+    if constexpr (DecShared<C, kLayWide>::NS > 1)
+        if (!two_slots) {
+            decode_uniform_kernel<C, kLayOne><<<a.d.W, C::NT, 0, s>>>(a);
+            return;
+        }
+    decode_uniform_kernel<C, kLayWide><<<a.d.W, C::NT, 0, s>>>(a);
 }
 template <class C>
 void launch_step(const StepArgs& a, hipStream_t s) {
@@ -1364,8 +1369,9 @@ hipError_t launch_decode_uniform(const UniArgs& a, int G, int hp, hipStream_t s)
     if (G != 1 && G != 2 && G != 4 && G != 8) return hipErrorInvalidValue;
     if (hp != 1 && (hp != 2 || a.d.Hkv % 2 != 0)) return hipErrorInvalidValue;
     if (a.d.W <= 0) return hipSuccess;
-    if (hp == 2) PD_DISPATCH(PairCfg, G, launch_u, a, s);
-    else PD_DISPATCH(BalCfg, G, launch_u, a, s);
+    const bool two = uniform_two_slots(a.per_wg, ((int64_t)a.chunk_tokens + kPage - 1) / kPage + 1);
+    if (hp == 2) PD_DISPATCH(PairCfg, G, launch_u, a, two, s);
+    else PD_DISPATCH(BalCfg, G, launch_u, a, two, s);
     return hipGetLastError();
 }
 

@@ -56,8 +56,8 @@ constexpr float kWScale = 32768.f;                       // scale of the weights
 constexpr float kLoScale = 2048.f;                       // and, on top, of their lower parts
 constexpr float kDecLn2 = 0.69314718055994531f;
 
-// LDS layouts: kLayWide holds two blocks per wave (one at G = 8); kLayOne one block and leaves room for
-// the device-range kernel's own arrays; kLayStep (the fused cascade step, so that a CU holds the
+// LDS layouts: kLayWide holds two blocks per wave (one at G = 8); kLayOne one block (the uniform split's
+// longer items, and the device-range kernel, whose own arrays it leaves room for); kLayStep (the fused cascade step, so that a CU holds the
 // workgroup beside a prefix workgroup, 80 KB each) one block, a shorter page list, one flush buffer,
 // and at G = 8 the flush in two passes.
 enum { kLayWide, kLayOne, kLayStep };

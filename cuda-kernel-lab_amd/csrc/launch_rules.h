@@ -39,6 +39,14 @@ inline UniformSplit uniform_split(int64_t chunks, int Hkv, int64_t cus, int64_t 
     return 4 * longest(two) <= 5 * longest(one) || 4 * two.W >= 3 * cus ? two : one;
 }
 
+// Whether a uniform-split workgroup at G <= 4 holds two 32-key blocks per wave in LDS (decode_body.h). A
+// second block in flight pays where it is all there is to start with, but its q rows then go through LDS
+// with every block. One / two, us: 8 x 8192 tokens 47.7 / 48.3, 1 x 32768 27.9 / 28.2, 33 of 66-333 13.3 /
+// 13.9, 65 of 666-3333 with 4 kv heads 71.6 / 74.5; with one item of up to 32 pages per workgroup two are
+// faster at G = 1 (32 kv heads: 2 of 66-333 7.04 / 6.76, 2 of 233-1166 9.55 / 9.34, 8 of 66-333 9.96 / 9.77)
+// and within 0.3 either way at G = 4.
+inline bool uniform_two_slots(int64_t per, int64_t pages_per_item) { return per == 1 && pages_per_item <= 32; }
+
 // Kv heads per workgroup of the device-range decode over `cus` CUs. Two heads stream faster but double the
 // ranges, and so the partials of every long sequence; the lengths are not known here, only that a sequence
 // attends at most per_seq pages. Two from 16 such pages per range on (about 8 real ones in a ragged batch,

@@ -16,6 +16,8 @@ void rule_uniform_split(int64_t chunks, int Hkv, int64_t cus, int64_t seg_max, i
     out[3] = u.W;
 }
 
+bool rule_uniform_two_slots(int64_t per, int64_t pages) { return pdattn::uniform_two_slots(per, pages); }
+
 int rule_device_range_heads(int64_t B, int64_t per_seq, int Hkv, int64_t cus) {
     return pdattn::device_range_heads(B, per_seq, Hkv, cus);
 }

@@ -67,6 +67,22 @@ def test_partials_keep_fp32_accuracy(Hq, Hkv):
     assert np.linalg.norm(po - ro) <= 4 * 2.0 ** -24 * np.sqrt(ct) * np.linalg.norm(ro)
 
 
+@pytest.mark.parametrize("chunk_tokens", [495, 497, 512])
+@pytest.mark.parametrize("Hq,Hkv", [(8, 8), (16, 8), (32, 8), (64, 8)], ids=["G1", "G2", "G4", "G8"])
+def test_uniform_partials_where_the_layout_changes(Hq, Hkv, chunk_tokens):
+    """Items of 32 and 33 pages, and two items per workgroup (36 x 8): one and two LDS blocks per wave;
+    unaligned starts."""
+    import _gpu
+    print(f"[case] uniform layouts Hq={Hq} Hkv={Hkv} chunk={chunk_tokens}", flush=True)
+    for lens in ([1200, 33, 700], [int(x) for x in range(480, 552, 2)]):
+        bt = inputs.make_batch(lens, Hq, Hkv, seed=79)
+        nc = 2 if bt.B == 3 else 1
+        ro, rl = oracle.partials(bt.q, bt.k, bt.v, bt.indptr, bt.indices, bt.last, Hq, Hkv, nc, chunk_tokens, 23)
+        po, pl = _gpu.run_partials(_gpu.DeviceBatch(bt), nc, chunk_tokens, 23)
+        check_lse(pl, rl, tag="partial lse")
+        assert np.linalg.norm(po - ro) <= 4 * 2.0 ** -24 * np.sqrt(chunk_tokens) * np.linalg.norm(ro)
+
+
 def test_infinite_values():
     """An infinite V makes its dim infinite in every head (its weight's low half must not turn it into
     NaN) and leaves the other dims alone."""

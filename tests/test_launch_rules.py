@@ -51,6 +51,16 @@ def test_two_heads_per_item_leave_no_more_of_the_chip_idle(rules):
     assert _uniform(rules, 64, 7)[0] == 1
 
 
+def test_uniform_split_slots(rules):
+    """Two blocks per wave only where a workgroup has one short item."""
+    def two(per, pages):
+        f = rules.rule_uniform_two_slots
+        f.restype = ctypes.c_bool
+        return f(ctypes.c_int64(per), ctypes.c_int64(pages))
+    assert [two(1, n) for n in (2, 32, 33, 129, 2048)] == [True, True, False, False, False]
+    assert not two(2, 2) and not two(24, 32)
+
+
 def test_device_ranges_of_short_batches_keep_one_head(rules):
     """Two heads only where every range holds enough pages, or there are more sequences than ranges."""
     def heads(B, longest, Hkv, cus=256):
