@@ -23,9 +23,10 @@
 // slot, reads all operands of the block into registers (K rows with ds_read_b128, V with the
 // transposing ds_read_b64_tr_b16), issues the next loads into the slot, the score MFMAs between them, and
 // computes. One slot keeps 16 KB per wave, 64 KB per CU, in flight, which covers the loaded latency of
-// long streams; two slots
-// (G <= 4) start short sequences sooner: one sequence of 4096 tokens 9.43 -> 8.93 us, 128 of 16-512
-// at G = 1 96.2 -> 94.6 us, 32768 tokens 27.6 -> 26.8 us; 64 x 1024 41.9 -> 42.1 us.
+// long streams; two slots (plans at G <= 4) start short sequences sooner: one sequence of 4096 tokens 9.43
+// -> 8.93 us, 32768 26.8 -> 26.2, 128 of 16-512 at G = 1 95.2 -> 94.5; 64 x 1024 41.9 -> 42.4. Over 100 ragged
+// batches of 2-200 sequences they are between 3% faster and 5% slower, and no size says which. The uniform
+// split, whose items are mostly longer, has its own rule (launch_rules.h).
 //
 // Bound: HBM (64 ragged sequences of 256-4096 tokens, 548 MB: 85 us at G = 4 and 87 us at G = 8 for
 // the decode launch, where one contiguous read of as many bytes takes 82 us). The vector-unit body
