@@ -1194,10 +1194,10 @@ __global__ __launch_bounds__(kMergeThreads) void merge_ranges_kernel(DevMergeArg
 
 // One kv head per workgroup (C::HP = 1), or HP neighbouring heads of a page-range plan: workgroup x
 // runs the plan's workgroups HP x .. HP x + HP - 1.
-template <class C, bool RANGES>
+template <class C, bool RANGES, int LAY = kLayWide>
 __global__ __launch_bounds__(C::NT, 1) void decode_balanced_kernel(BalArgs a) {
-    __shared__ DecShared<C, kLayWide> S;
-    balanced_body<C, false, kLayWide, RANGES>(a, S, blockIdx.x);
+    __shared__ DecShared<C, LAY> S;
+    balanced_body<C, false, LAY, RANGES>(a, S, blockIdx.x);
 }
 
 // The reference-shaped uniform split on the balanced body (items of equal key ranges, descriptors
@@ -1267,6 +1267,11 @@ void launch_b(const BalArgs& a, hipStream_t s) {
 }
 template <class C>
 void launch_pair(const BalArgs& a, hipStream_t s) {
+    if constexpr (DecShared<C, kLayWide>::NS > 1)
+        if (plan_one_slot(a.B, a.nnz, a.ngroups, C::G)) {
+            decode_balanced_kernel<C, true, kLayOne><<<a.W / C::HP, C::NT, 0, s>>>(a);
+            return;
+        }
     decode_balanced_kernel<C, true><<<a.W / C::HP, C::NT, 0, s>>>(a);
 }
 template <class C>

@@ -24,9 +24,8 @@
 // transposing ds_read_b64_tr_b16), issues the next loads into the slot, the score MFMAs between them, and
 // computes. One slot keeps 16 KB per wave, 64 KB per CU, in flight, which covers the loaded latency of
 // long streams; two slots (plans at G <= 4) start short sequences sooner: one sequence of 4096 tokens 9.43
-// -> 8.93 us, 32768 26.8 -> 26.2, 128 of 16-512 at G = 1 95.2 -> 94.5; 64 x 1024 41.9 -> 42.4. Over 100 ragged
-// batches of 2-200 sequences they are between 3% faster and 5% slower, and no size says which. The uniform
-// split, whose items are mostly longer, has its own rule (launch_rules.h).
+// -> 8.93 us, 32768 26.8 -> 26.2, 128 of 16-512 at G = 1 95.2 -> 94.5; 64 x 1024 41.9 -> 42.4. Which batches
+// run with one, and the uniform split's rule: launch_rules.h.
 //
 // Bound: HBM (64 ragged sequences of 256-4096 tokens, 548 MB: 85 us at G = 4 and 87 us at G = 8 for
 // the decode launch, where one contiguous read of as many bytes takes 82 us). The vector-unit body
@@ -57,8 +56,8 @@ constexpr float kWScale = 32768.f;                       // scale of the weights
 constexpr float kLoScale = 2048.f;                       // and, on top, of their lower parts
 constexpr float kDecLn2 = 0.69314718055994531f;
 
-// LDS layouts: kLayWide holds two blocks per wave (one at G = 8); kLayOne one block (the uniform split's
-// longer items, and the device-range kernel, whose own arrays it leaves room for); kLayStep (the fused cascade step, so that a CU holds the
+// LDS layouts: kLayWide holds two blocks per wave (one at G = 8); kLayOne one block (where that is faster,
+// and the device-range kernel, whose own arrays it leaves room for); kLayStep (the fused cascade step, so that a CU holds the
 // workgroup beside a prefix workgroup, 80 KB each) one block, a shorter page list, one flush buffer,
 // and at G = 8 the flush in two passes.
 enum { kLayWide, kLayOne, kLayStep };

@@ -47,6 +47,21 @@ inline UniformSplit uniform_split(int64_t chunks, int Hkv, int64_t cus, int64_t 
 // and within 0.3 either way at G = 4.
 inline bool uniform_two_slots(int64_t per, int64_t pages_per_item) { return per == 1 && pages_per_item <= 32; }
 
+// Whether a plan of two kv heads per workgroup at G <= 4 holds one block per wave instead. One is faster where
+// a range holds a few blocks per wave, of several sequences; its q rows then come to registers once per
+// segment, which very short segments wait for, the more heads the longer. So: at least 12 sequences, at most
+// 64 pages per range, and at least 4 pages per sequence at G <= 2, 20 at G = 4. One / two, us: G = 4, 64 x 1024
+// tokens 41.8 / 42.4, 20 of 300-1000 with 16 kv heads 25.0 / 25.8, but 64 of 7-224 15.8 / 15.5 and 64 of 11-67
+// 15.8 / 15.2; G = 2, 32 of 300-1000 20.2 / 20.8, 128 of 7-224 19.8 / 20.4; G = 1, 37 of 18-432 with 16 kv heads
+// 18.0 / 18.7 (18.0 with the vector-unit body), 32 of 7-224 with 32 19.2 / 20.3, but 200 of 11-67 41.4 / 40.8.
+// Past 64 pages two are as fast or faster at G = 1 (128 of 16-512 with 32 kv heads, 131 pages, 95.2 / 94.5)
+// and within 0.6% at G = 2 and 4; of fewer sequences some are faster with two (6 of 512-2560 13.7 / 13.4, 1 x
+// 32768 26.8 / 26.2) and with one head per workgroup as many lose as gain (12 of 18-432, 16 kv heads, 12.1 /
+// 11.7).
+inline bool plan_one_slot(int64_t B, int64_t nnz, int64_t ngroups, int G) {
+    return B >= 12 && nnz <= 64 * ngroups && nnz >= (G <= 2 ? 4 : 20) * B;
+}
+
 // Kv heads per workgroup of the device-range decode over `cus` CUs. Two heads stream faster but double the
 // ranges, and so the partials of every long sequence; the lengths are not known here, only that a sequence
 // attends at most per_seq pages. Two from 16 such pages per range on (about 8 real ones in a ragged batch,

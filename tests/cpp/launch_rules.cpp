@@ -18,6 +18,10 @@ void rule_uniform_split(int64_t chunks, int Hkv, int64_t cus, int64_t seg_max, i
 
 bool rule_uniform_two_slots(int64_t per, int64_t pages) { return pdattn::uniform_two_slots(per, pages); }
 
+bool rule_plan_one_slot(int64_t B, int64_t nnz, int64_t ngroups, int G) {
+    return pdattn::plan_one_slot(B, nnz, ngroups, G);
+}
+
 int rule_device_range_heads(int64_t B, int64_t per_seq, int Hkv, int64_t cus) {
     return pdattn::device_range_heads(B, per_seq, Hkv, cus);
 }

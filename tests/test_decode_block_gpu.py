@@ -67,6 +67,23 @@ def test_partials_keep_fp32_accuracy(Hq, Hkv):
     assert np.linalg.norm(po - ro) <= 4 * 2.0 ** -24 * np.sqrt(ct) * np.linalg.norm(ro)
 
 
+@pytest.mark.parametrize("Hq", [8, 16, 32, 64], ids=["G1", "G2", "G4", "G8"])
+def test_paired_plans_with_one_and_two_blocks_per_wave(Hq):
+    """Two kv heads per workgroup, block edges and poison: 36 short sequences (6 pages each: one LDS block per
+    wave at G <= 2), 30 with long ones among them (26 pages each: one), 16 longer ones and 11 (two)."""
+    import _gpu
+    print(f"[case] paired plans Hq={Hq}", flush=True)
+    long = [1000 - 13 * i for i in range(12)]
+    for lens in (LENS * 2, LENS + long, [5000 - 77 * i for i in range(16)], [900 + i for i in range(11)]):
+        bt = inputs.make_batch(lens, Hq, 8, seed=80)
+        ro, rl = oracle.decode(bt.q, bt.k, bt.v, bt.indptr, bt.indices, bt.last, Hq, 8, threads=8)
+        _poison(bt)
+        o, l, info = _gpu.run_plan(_gpu.DeviceBatch(bt))
+        assert info.paired == 1
+        check_out(o, ro, tag=f"{len(lens)} sequences")
+        check_lse(l, rl, tag=f"{len(lens)} sequences")
+
+
 @pytest.mark.parametrize("chunk_tokens", [495, 497, 512])
 @pytest.mark.parametrize("Hq,Hkv", [(8, 8), (16, 8), (32, 8), (64, 8)], ids=["G1", "G2", "G4", "G8"])
 def test_uniform_partials_where_the_layout_changes(Hq, Hkv, chunk_tokens):

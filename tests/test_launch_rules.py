@@ -61,6 +61,19 @@ def test_uniform_split_slots(rules):
     assert not two(2, 2) and not two(24, 32)
 
 
+def test_plan_slots(rules):
+    """One block per wave for 12 and more sequences of 4 (G <= 2) or 20 pages and more each, up to 64 pages
+    per range."""
+    def one(B, nnz, ngroups, G):
+        f = rules.rule_plan_one_slot
+        f.restype = ctypes.c_bool
+        return f(ctypes.c_int64(B), ctypes.c_int64(nnz), ctypes.c_int64(ngroups), G)
+    for G, least in ((1, 4), (2, 4), (4, 20)):
+        assert [one(B, 30 * B, 32, G) for B in (1, 11, 12, 60)] == [False, False, True, True]
+        assert one(64, 64 * 64, 64, G) and not one(64, 64 * 64 + 1, 64, G)
+        assert one(64, least * 64, 64, G) and not one(64, least * 64 - 1, 64, G)
+
+
 def test_device_ranges_of_short_batches_keep_one_head(rules):
     """Two heads only where every range holds enough pages, or there are more sequences than ranges."""
     def heads(B, longest, Hkv, cus=256):
